@@ -100,8 +100,9 @@ struct det_ctx {
     return gemm_planes;
   }
   // The MFMA attention's work area for a (null where that form does not
-  // apply or would need more than kAttnWorkMax bytes: the vector-ALU kernel
-  // runs then).
+  // apply or would need more than kAttnWorkMax bytes even in query chunks: the
+  // vector-ALU kernel runs then, and also for a call whose unchunked form
+  // passes the bound when a recording stream keeps the area from growing).
   static constexpr uint64_t kAttnWorkMax = uint64_t(512) << 20;
   void attach_attn_work(det::AttnArgs& a) {
     const uint64_t bytes = det::attn_mfma_bytes(a);
@@ -109,6 +110,7 @@ struct det_ctx {
     a.work_bytes = 0;
     if (bytes == 0 || bytes > kAttnWorkMax) return;
     if (bytes > attn_work_bytes) {
+      if (capturing && det::attn_mfma_unchunked_bytes(a) > kAttnWorkMax) return;
       grow_check("attention");
       HIPC(hipStreamSynchronize(stream));
       if (attn_work) HIPC(hipFree(attn_work));

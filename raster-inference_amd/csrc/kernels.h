@@ -264,14 +264,32 @@ bool launch_attention_mfma(const AttnArgs& a, void* work, uint64_t work_bytes, h
 struct AttnMfmaArgs;
 // The MFMA form's layout of a.work (false where the form does not apply).
 bool attn_mfma_plan(const AttnArgs& a, AttnMfmaArgs& m);
+// What the work area would take without query chunks (0 as attn_mfma_bytes).
+uint64_t attn_mfma_unchunked_bytes(const AttnArgs& a);
 // MFMA operand limb blocks of Q / K rows (one 1 KB block per 16-row tile,
-// 64-dim substep and limb: lane 16 g + i holds row i, dims [64 s + 16 g, +16)
-// as bytes j of x ^ 0x808080, the four-limb split x = sum_j c_j 256^j + C4).
+// 64-dim substep and limb: lane 16 g + i holds row i, dims [64 s + 16 g, +16)).
+// A row with a value outside [-2^23, 2^23) is wide: bytes j of x ^ 0x808080,
+// the four-limb split x = sum_j c_j 256^j + C4. Any other row is narrow: bytes
+// j of (x + 2^23) ^ 0x808080, x = sum_{j<3} c_j 256^j + C3, with a zero fourth
+// limb.
 constexpr int64_t kAttnC4 = 8421504;
+constexpr int64_t kAttnC3 = 32896;
 constexpr uint32_t kAttnOp = 1024;
+// Whether any of 16 values needs the wide split.
+__device__ inline bool attn_wide16(const int32_t (&x)[16]) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) m |= (uint32_t(x[e]) + 0x800000u) & 0xff000000u;
+  return m != 0;
+}
+// A row's sum of x - C (below 2^62 in magnitude) and its width in one word.
+__host__ __device__ inline int64_t attn_pack_sum(int64_t sum, bool wide) {
+  return int64_t(uint64_t(sum) << 1) | int64_t(wide);
+}
 // 16 consecutive values of a row -> limb j's 16 bytes as four words w[j][0..3]
-// (byte j of x ^ 0x808080, four values per word) and the sum of x - C4
-__device__ inline int64_t attn_split16(const int32_t (&x)[16], uint32_t (&w)[4][4]) {
+// (four values per word) and the sum of x - C
+__device__ inline int64_t attn_split16(const int32_t (&x)[16], bool wide, uint32_t (&w)[4][4]) {
+  const uint32_t bias = wide ? 0u : 0x800000u;
   int64_t s = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
@@ -279,12 +297,12 @@ __device__ inline int64_t attn_split16(const int32_t (&x)[16], uint32_t (&w)[4][
     for (int d = 0; d < 4; ++d) w[j][d] = 0;
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
-    const uint32_t u = uint32_t(x[e]) ^ 0x00808080u;
-    s += int64_t(x[e]) - kAttnC4;
+    const uint32_t u = (uint32_t(x[e]) + bias) ^ 0x00808080u;
+    s += int64_t(x[e]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) w[j][e >> 2] |= ((u >> (8 * j)) & 0xffu) << (8 * (e & 3));
   }
-  return s;
+  return s - 16 * (wide ? kAttnC4 : kAttnC3);
 }
 struct AttnMfmaArgs {
   uint32_t hd, groups;
@@ -298,9 +316,16 @@ struct AttnMfmaArgs {
   int64_t* qsum;
   int64_t* ksum;
   int64_t* vblk;
+  uint32_t* vwide;  // per KV head and key substep: the V limbs take the four-limb split
+  const int32_t* v;
+  uint64_t kv_ld;
+  // the chunk of queries [t0, t0 + crow_used) whose scores (crow rows per
+  // head) are in the work area
+  uint64_t t0, crow, crow_used;
   int32_t* scores;
-  int32_t* resid;
+  int32_t* extra;  // per (head, query)
   uint32_t* argm;
+  uint32_t* wtot;
 };
 
 // Elementwise ops (saturating Q16.16).

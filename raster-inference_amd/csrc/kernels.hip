@@ -1914,27 +1914,8 @@ __global__ __launch_bounds__(256) void k_head_norm_rope(HeadNormRope a) {
   // One 16-dim slot of the 1 KB MFMA operand blocks of head row hidx (of the q
   // or k blocks): dims [16 sl, 16 sl + 16) go to limb j's block
   // ((hidx * nt + t / 16) * nsub + sl / 4) * 4 + j, bytes (16 (sl % 4) + t % 16) * 16;
-  // returns the slot's sum of x - C4 (src null: a padding row, x = C4)
-  auto put_slot = [&](int8_t* limbs, uint64_t nt, uint32_t hidx, uint32_t sl, const int32_t* src) {
-    int32_t x16[16];
-    if (src) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int4 v = reinterpret_cast<const int4*>(src + 16 * sl)[q];
-        x16[4 * q] = v.x, x16[4 * q + 1] = v.y, x16[4 * q + 2] = v.z, x16[4 * q + 3] = v.w;
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < 16; ++q) x16[q] = int32_t(kAttnC4);
-    }
-    uint32_t w[4][4];
-    const int64_t sm = attn_split16(x16, w);
-    int8_t* blk = limbs + ((uint64_t(hidx) * nt + t / 16) * nsub + sl / 4) * 4 * kAttnOp + (16 * (sl % 4) + t % 16) * 16;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<uint4*>(blk + j * kAttnOp) = make_uint4(w[j][0], w[j][1], w[j][2], w[j][3]);
-    return sm;
-  };
+  // returns the row's packed sum of x - C (src null: a padding row, x = C3). Every
+  // lane takes part: a row is wide when any of its slots has a wide value.
   // sum over the spr lanes of a row's slots (every lane takes part): segments
   // of a power-of-two width share the wave, any other width takes one row per
   // pass and the whole wave (lanes past its slots add zero)
@@ -1946,8 +1927,36 @@ __global__ __launch_bounds__(256) void k_head_norm_rope(HeadNormRope a) {
     for (uint32_t off = 1; off < spr; off <<= 1) sm += __shfl_xor(sm, int(off), 64);
     return sm;
   };
+  // whether any slot of the lane's row has `w` set (every lane takes part)
+  auto seg_any = [&](bool w) {
+    const uint64_t b = __ballot(w);
+    return pow2 ? ((b >> (lane & ~(spr - 1))) & ((uint64_t(1) << spr) - 1)) != 0 : b != 0;
+  };
+  auto put_slot = [&](bool on, int8_t* limbs, uint64_t nt, uint32_t hidx, uint32_t sl, const int32_t* src) {
+    int32_t x16[16];
+    if (on && src) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int4 v = reinterpret_cast<const int4*>(src + 16 * sl)[q];
+        x16[4 * q] = v.x, x16[4 * q + 1] = v.y, x16[4 * q + 2] = v.z, x16[4 * q + 3] = v.w;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) x16[q] = int32_t(kAttnC3);
+    }
+    const bool wide = seg_any(attn_wide16(x16));
+    uint32_t w[4][4];
+    const int64_t sm = attn_split16(x16, wide, w);
+    if (on) {
+      int8_t* blk = limbs + ((uint64_t(hidx) * nt + t / 16) * nsub + sl / 4) * 4 * kAttnOp + (16 * (sl % 4) + t % 16) * 16;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<uint4*>(blk + j * kAttnOp) = make_uint4(w[j][0], w[j][1], w[j][2], w[j][3]);
+    }
+    return attn_pack_sum(seg_sum(on ? sm : 0), wide);
+  };
   auto put_blocks = [&](int8_t* limbs, int64_t* sums, uint64_t nt, uint32_t hidx, const int32_t* src) {
-    const int64_t sm = seg_sum(lane < spr ? put_slot(limbs, nt, hidx, lane, src) : 0);
+    const int64_t sm = put_slot(lane < spr, limbs, nt, hidx, lane, src);
     if (lane == 0) sums[uint64_t(hidx) * nt * 16 + t] = sm;
   };
   if (t >= a.rows) {
@@ -2059,10 +2068,8 @@ __global__ __launch_bounds__(256) void k_head_norm_rope(HeadNormRope a) {
         const uint32_t r = r0 + 4 * u;
         const bool on = lane < rpp * spr && u < RPW && ((blk_mask >> u) & 1u);
         const bool is_q = r < a.nh;
-        int64_t sm = 0;
-        if (on) sm = is_q ? put_slot(a.qlimbs, a.nqt, r, sl, rowbuf[wave][u])
-                          : put_slot(a.klimbs, a.nkt, r - a.nh, sl, rowbuf[wave][u]);
-        sm = seg_sum(sm);
+        const int64_t sm = put_slot(on, is_q ? a.qlimbs : a.klimbs, is_q ? a.nqt : a.nkt, is_q ? r : r - a.nh, sl,
+                                    rowbuf[wave][u < RPW ? u : 0]);
         if (on && sl == 0) {
           if (is_q) a.qsum[uint64_t(r) * a.nqt * 16 + t] = sm;
           else a.ksum[uint64_t(r - a.nh) * a.nkt * 16 + t] = sm;

@@ -223,6 +223,44 @@ def test_attention_causal(ctx, nq, nh, nkv, hd, window, mag):
     assert np.array_equal(out.numpy(), oracle_attention(q, k, v, nq, nq, nh, nkv, hd, window))
 
 
+@pytest.mark.parametrize("nq,nrows,nh,nkv,hd,window,wide", [
+    (16, 16, 4, 1, 64, 0, False),       # one tile of queries and keys
+    (31, 47, 3, 1, 64, 0, False),       # three heads per KV head, rows past the queries
+    (515, 515, 8, 2, 256, 100, False),  # one key past a score span; windows that start inside a substep
+    (2300, 2300, 8, 2, 256, 0, True),   # two chunks of queries, more than 2048 keys, two key tiles per wave
+    (1100, 1100, 8, 4, 128, 1030, True),
+])
+def test_attention_causal_tiles(ctx, nq, nrows, nh, nkv, hd, window, wide):
+    """Normalised rows (three limbs) with single rows, keys and values past 24 bits (`wide`, int32
+    extremes among them), a query whose softmax is one key of weight 65536, and equal maxima."""
+    rng = np.random.default_rng(nq + hd)
+    q, k, v = (np.rint(rng.normal(size=(n, h * hd)) * 65536).astype(np.int32)
+               for n, h in ((nq, nh), (nrows, nkv), (nrows, nkv)))
+    k[3], v[5, :hd] = k[2], -65536
+    q[9] = np.tile(k[4, :hd], nh) * 3  # its own key far above the rest
+    if wide:
+        k[70, 5], k[900, 7], v[130, 3], v[700, 1], q[300, 2] = 1 << 23, -(1 << 31), (1 << 31) - 1, -(1 << 24), 1 << 25
+    out = ctx.empty((nq, nh * hd))
+    ctx.attention(ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), nq, nrows, nh, nkv, hd, window, out)
+    got, L, g = out.numpy(), oracle_lib.lib(), nh // nkv
+    picks = {0, 9, 15, nq - 1, nq // 2, 70, 71, 300, 901, 1023, 1050, 2047, 2048}
+    for t in sorted(x for x in picks if x < nq):
+        start = max(0, t + 1 - window) if window else 0
+        for h in range(nh):
+            cols = slice(h // g * hd, (h // g + 1) * hd)
+            ks, vs = np.ascontiguousarray(k[start:t + 1, cols]), np.ascontiguousarray(v[start:t + 1, cols])
+            qs = np.ascontiguousarray(q[t, h * hd:(h + 1) * hd])
+            logits = np.zeros(len(ks), dtype=np.int32)
+            for r in range(len(ks)):
+                o = oracle_lib.C.c_int32()
+                L.orc_attention_score(oracle_lib.ptr(qs), oracle_lib.ptr(ks[r]), hd, oracle_lib.C.byref(o))
+                logits[r] = o.value
+            w, o = np.empty_like(logits), np.empty(hd, dtype=np.int32)
+            L.orc_attention_softmax(oracle_lib.ptr(logits), len(ks), oracle_lib.ptr(w))
+            L.orc_attention_weighted_sum(oracle_lib.ptr(w), oracle_lib.ptr(vs), len(ks), hd, oracle_lib.ptr(o))
+            assert np.array_equal(got[t, h * hd:(h + 1) * hd], o), (t, h)
+
+
 @pytest.mark.parametrize("n", [1, 5, 1023, 1024, 1025, 262144])
 def test_argmax_first(ctx, n):
     rng = np.random.default_rng(n)
