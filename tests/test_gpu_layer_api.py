@@ -237,3 +237,58 @@ def test_kv_handle_smaller_than_window_fails_closed(ctx):
     for pos in range(5, 12):
         ops.layer_decode(0, row, None, ring, None, pos, row)
     assert ring.info()[0] == 8
+
+
+class _Shifted:
+    """A device buffer's view `words` int32 past its start (not 16-byte aligned)."""
+
+    def __init__(self, buf, words=1):
+        self.buf, self.ptr = buf, buf.ptr + 4 * words
+
+
+@pytest.mark.parametrize("prompt,window,donor", [(1, 24, False), (40, 24, False), (70, 512, False), (700, 40, True)])
+def test_layer_decode_routes_agree(ctx, prompt, window, donor):
+    """det_layer_decode on the fused step's kernels (aligned rows, the cache's next position) against the
+    per-op form (rows off alignment), for sliding rings past their wrap, full and donor caches: the same
+    rows and the same cache contents, step after step; a position other than the cache's length takes the
+    per-op form and the next fused step still agrees."""
+    cfg = synthetic.e4b_config(layers=4, vocab=512, sliding_window=window)
+    if donor:
+        cfg["text_config"]["num_kv_shared_layers"] = 2
+    model = rd.Model(ctx, cfg)
+    for name, v, s in synthetic.synthetic_model_fast(cfg, 3, scale_max=256):
+        model.set_tensor(name, v, s)
+    model.finalize()
+    H, tc = 2560, cfg["text_config"]
+    rng = np.random.default_rng(prompt)
+    rows = np.rint(rng.normal(size=(prompt, H)) * 4 * 65536).astype(np.int32)
+    steps = [np.rint(rng.normal(size=H) * 4 * 65536).astype(np.int32) for _ in range(5)]
+
+    def play(shift: bool):
+        ops = rd.LayerOps(model)
+        caches = {l: rd.KvCache(model, l, prompt + 8) for l in range(4) if donor_of(tc, l) is None}
+        x, out = ctx.to_device(rows), ctx.empty((prompt, H))
+        for l in caches:
+            ops.layer_prefill(l, x, prompt, None, None, caches[l], out)
+        got = []
+        for i, row in enumerate(steps):
+            pos = prompt + i
+            buf, res = ctx.empty(H + 1), ctx.empty(H + 1)
+            src, dst = (_Shifted(buf), _Shifted(res)) if shift else (buf, res)
+            buf.upload(np.concatenate([np.zeros(int(shift), np.int32), row, np.zeros(1 - int(shift), np.int32)]))
+            for l in range(4):
+                d = donor_of(tc, l)
+                rope = pos + (7 if i == 2 and d is None and l == 0 else 0)
+                ops.layer_decode(l, src, None, caches.get(l), None if d is None else caches[d], rope, dst)
+                got.append(res.numpy()[int(shift):H + int(shift)].copy())
+            if i == 3:  # in place
+                ops.layer_decode(3 if not donor else 1, src, None, caches.get(3 if not donor else 1), None,
+                                 pos + 1, src)
+                got.append(buf.numpy()[int(shift):H + int(shift)].copy())
+                break
+        return got, [c.read_logical() for c in caches.values()]
+
+    a, b = play(False), play(True)
+    assert len(a[0]) == len(b[0]) and all(np.array_equal(p, q) for p, q in zip(a[0], b[0]))
+    for (k0, v0), (k1, v1) in zip(a[1], b[1]):
+        assert np.array_equal(k0, k1) and np.array_equal(v0, v1)
