@@ -270,6 +270,15 @@ def test_argmax_first(ctx, n):
     assert ctx.argmax_first(ctx.to_device(x), n) == int(np.argmax(x))
 
 
+def test_tanh_over_its_whole_rational_range(ctx):
+    """A softcap of 1.0 is tanh itself: every argument around the rational's range, both signs."""
+    x = np.arange(-196700, 196701, dtype=np.int32)
+    d = ctx.to_device(x)
+    ctx.elementwise(rd.DET_EW_SOFTCAP, d, None, x.size, 1 << 16)
+    f = oracle_lib.lib().orc_tanh_act
+    assert np.array_equal(d.numpy(), np.array([f(int(a)) for a in x], dtype=np.int32))
+
+
 @pytest.mark.parametrize("n", [3, 5000, 5003, 20483])
 def test_elementwise_ops(ctx, n):
     # (n % 4 != 0: the quad-vector GELU kernel's scalar tail)
