@@ -139,10 +139,11 @@ def test_i16_e4b_shaped_model_takes_the_fused_step(i16_two_layers):
     assert gm.fused_decode
 
 
-@pytest.mark.parametrize("prompt_len", [9, 100])
+@pytest.mark.parametrize("prompt_len", [9, 100, 193])
 def test_i16_e4b_shaped_capture_matches_oracle(i16_two_layers, prompt_len):
     # prefill (GEMV under 16 rows, MFMA GEMMs with the fused q/k/v and the
-    # gate/up GELU epilogue above), then the fused decode step graph-replayed
+    # gate/up GELU epilogue above, in its large-wave form past 128 rows), then
+    # the fused decode step graph-replayed
     _, (om, gm) = i16_two_layers
     prompt = np.random.default_rng(prompt_len).integers(0, 4096, size=prompt_len).tolist()
     exp = om.capture(prompt, 12)
