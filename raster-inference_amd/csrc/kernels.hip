@@ -3131,8 +3131,13 @@ static bool gemm_small(const DevMatrix& W, uint64_t m) {
 //   32 tokens x 48 rows, 6 waves (96 KB): q/k/v 3072 x 2560 11.7 against
 //     14.4 us in 384 16 x 64 blocks;
 //   16 tokens x 80 rows, 5 waves (80 KB): o 2560 x 2048 8.5 against 9.3 us.
+// Ahead of them, on ten waves of one token group and four buffers, for the
+// row counts below the first shape's (20480-row gate/up with its limb
+// expansion, against 128 x 128 blocks): 32 tokens x 80 rows at 17 to 32 rows,
+// 20.4 -> 17.9 us; 32 tokens x 160 rows at 33 to 64, 24.8 -> 22.4 us (64 x 80
+// on four waves 29.6 us: each reads eight operands for fifteen MFMAs).
 // At 512 and 2048 rows the grids take several rounds and none applies.
-enum class PadShape { kNone, k64x160, k32x48, k16x80 };
+enum class PadShape { kNone, k64x160, k32x48, k16x80, k32x80, k32x160 };
 static PadShape gemm_pad_shape(const DevMatrix& W, uint64_t m) {
   if (W.storage != kInt8 || W.planes != 1 || W.kpad > 32 * 128) return PadShape::kNone;
   const uint64_t tiles = (W.rows + 15) / 16, cus = device_cus();
@@ -3140,6 +3145,8 @@ static PadShape gemm_pad_shape(const DevMatrix& W, uint64_t m) {
     const uint64_t blocks = ((m + tokens - 1) / tokens) * ((tiles + tb - 1) / tb);
     return blocks <= cus && blocks * 10 >= cus * 9;
   };
+  if (m > 16 && m <= 32 && fills(32, 5)) return PadShape::k32x80;
+  if (m > 32 && m <= 64 && fills(32, 10)) return PadShape::k32x160;
   if (fills(64, 10)) return PadShape::k64x160;
   if (fills(32, 3)) return PadShape::k32x48;
   if (fills(16, 5)) return PadShape::k16x80;
@@ -3153,6 +3160,10 @@ static void launch_gemm_pad(PadShape p, const DevMatrix& W, uint64_t m, int32_t*
     launch_gemm_lds_dg<16, 10, 4, 2, 8, 2, SPLIT, GELU, false>(W, m, out, ld_out, acc_out, a_tiled, a_tiles, s, split, {});
   else if (p == PadShape::k32x48)
     launch_gemm_lds_dg<8, 3, 2, 3, 8, 4, SPLIT, GELU, false>(W, m, out, ld_out, acc_out, a_tiled, a_tiles, s, split, {});
+  else if (p == PadShape::k32x80)
+    launch_gemm_lds_dg<8, 5, 2, 5, 8, 4, SPLIT, GELU, false>(W, m, out, ld_out, acc_out, a_tiled, a_tiles, s, split, {});
+  else if (p == PadShape::k32x160)
+    launch_gemm_lds_dg<8, 10, 2, 5, 8, 4, SPLIT, GELU, false>(W, m, out, ld_out, acc_out, a_tiled, a_tiles, s, split, {});
   else
     launch_gemm_lds_dg<4, 5, 1, 5, 8, 4, SPLIT, GELU, false>(W, m, out, ld_out, acc_out, a_tiled, a_tiles, s, split, {});
 }

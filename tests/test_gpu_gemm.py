@@ -150,7 +150,8 @@ def test_gemm_unaligned_activation_rows(ctx):
 @pytest.mark.parametrize("m,n,k", [(128, 3072, 2560), (100, 3072, 2560), (97, 3072, 2560), (64, 2560, 10240),
                                    (48, 2560, 2048), (128, 2560, 2048), (113, 2560, 2048), (256, 16384, 512),
                                    (300, 13100, 2600), (128, 20480, 2560), (100, 20480, 2560), (65, 20480, 2560),
-                                   (160, 16384, 2560)])
+                                   (160, 16384, 2560), (17, 20480, 2560), (32, 20475, 2560), (33, 20480, 2500),
+                                   (64, 20480, 4096)])
 def test_gemm_e4b_shapes_match_gemv_rows(ctx, m, n, k):
     q, s = synthetic.fast_int8_matrix(n * 31 + k, n, k, 256)
     acts = act_slab(m, k, seed=n + k)
