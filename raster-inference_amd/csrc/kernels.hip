@@ -1395,23 +1395,200 @@ __global__ __launch_bounds__(NT) void k_act_limbs_rows(const int32_t* __restrict
   }
 }
 
-// The GEMM kernels' epilogue: constant terms, digit planes, row scales, and
-// the output form (requantized rows, split rows, the GELU product, raw
-// accumulators, or a K range's partial plane). GELU: W holds tiles of 8 gate
-// rows and the matching 8 up rows (rows 16 t + i, i < 8: gate row 8 t + i;
-// rows 16 t + 8 + i: up row 8 t + i) and out[token][8 t + i] =
-// mul_sat(gelu(gate), up) (the decode step's gate/up epilogue; no other
-// output form).
-template <int FA, int FB, int NG, bool SPLIT, bool GELU>
-__device__ __forceinline__ void gemm_epilogue(const v4i (&acc)[FA][FB], uint64_t at0, uint64_t bt0, uint32_t wm,
-                                              uint32_t wn, uint32_t lane, int lp, const uint64_t (&gmask)[NG], bool many,
-                                              uint64_t parts, uint32_t chunk, const int32_t (&ep_rowsum)[FB],
-                                              const int32_t (&ep_scale)[FB], const int32_t* __restrict__ rowsum_p,
-                                              uint64_t rowsum_p_ld, uint64_t n_rows, uint64_t m_tokens,
-                                              int32_t* __restrict__ out, uint64_t ld_out, int64_t* __restrict__ acc_out,
-                                              const RowSplit& split, const KSplit& ks) {
+// Block: TA A tiles (TA / 4 token groups of 16 tokens, four limb tiles each)
+// x TB weight tiles on WM x WN waves, each wave (TA / WM) x (TB / WN) MFMA
+// tiles (whole token groups). A block whose token groups all take three limbs
+// multiplies no fourth-limb tile, and with two buffers does not copy them
+// either (with more, every wave copies a fixed number of tile-step halves per
+// step, so that one vmcnt immediate covers the steps in flight). Every
+// 128-column K step, the block's
+// TA + TB tile-steps (2 KB each) are copied straight from global memory into
+// one of NBUF LDS buffers with global_load_lds_dwordx4 (no register staging).
+// The 2 (TA + TB) copy halves are dealt out LPW per wave; where they do not
+// divide evenly, the slots past them re-copy the block's first weight
+// tile-step half into the buffer's spare kilobytes, so that every wave issues
+// the same copies per step:
+// the copies of the next NBUF - 1 steps are in flight while step s's MFMAs
+// run, and one barrier per step hands a buffer over. Copy h of a tile-step
+// takes the 16-byte half h of every lane's 32 columns (a weight tile-step's
+// contiguous half h; bytes [16 h, 16 h + 16) of each 32-byte slot of an
+// activation tile-step), so each 1 KB LDS half holds one MFMA operand of all
+// 64 lanes contiguously
+// and the 128-bit operand reads do not conflict on LDS banks. The MFMAs of a
+// step run as two passes over the wave's tile pairs (first 64 columns, then
+// the second 64), so consecutive MFMAs never share an accumulator.
+// GELU: W holds tiles of 8 gate rows and the matching 8 up rows (rows
+// 16 t + i, i < 8: gate row 8 t + i; rows 16 t + 8 + i: up row 8 t + i) and
+// out[token][8 t + i] = mul_sat(gelu(gate), up) (the decode step's gate/up
+// epilogue; no other output form).
+template <int TA, int TB, int WM, int WN, uint32_t GM, int NBUF, bool SPLIT, bool GELU, bool DG>
+__global__ __launch_bounds__(64 * WM * WN) void k_gemm_lds(const int8_t* __restrict__ a, const int8_t* __restrict__ q,
+                                                           const int32_t* __restrict__ scale,
+                                                           const int32_t* __restrict__ rowsum,
+                                                           const int32_t* __restrict__ rowsum_p, uint64_t rowsum_p_ld,
+                                                           uint64_t n_rows, uint64_t kpad, uint64_t m_tokens,
+                                                           uint64_t a_tiles, const uint32_t* __restrict__ a_flags,
+                                                           uint32_t mblocks, int32_t* __restrict__ out,
+                                                           uint64_t ld_out, int64_t* __restrict__ acc_out,
+                                                           RowSplit split, KSplit ks, int lp_arg) {
+  const int lp = DG ? lp_arg : 0;  // (single-plane instances fold it to 0)
+  constexpr int NW = WM * WN;                  // waves
+  constexpr int TS = TA + TB;                  // tile-steps per K step
+  constexpr int LPW = (2 * TS + NW - 1) / NW;  // 1 KB wave copies per wave per K step
+  constexpr int SLOTS = LPW * NW;               // 1 KB copy slots per LDS buffer (>= 2 TS)
+  constexpr int FA = TA / WM, FB = TB / WN;    // MFMA tiles per wave
+  static_assert(FA % 4 == 0 && NBUF >= 2, "whole token groups per wave");
+  extern __shared__ __attribute__((aligned(16))) int8_t lds_gemm[];
+  // the wave index as a scalar, so that copy addresses and LDS targets stay in SGPRs
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Block order: block b runs on XCD b % 8, and each XCD takes a contiguous
+  // range of logical blocks; logical blocks go in groups of GM m-blocks x all
+  // n-blocks with m fastest, so the blocks resident on one XCD at a time form
+  // a compact GM x (resident / GM) patch whose A and weight tiles share its L2.
+  // With K split into ks.chunks ranges, chunk c takes logical blocks
+  // [c nblk, (c + 1) nblk) and the same ordering inside them.
+  const uint32_t nall = gridDim.x, nblk = nall / ks.chunks;
+  uint32_t logical = blockIdx.x;
+  if (nall % 8 == 0) logical = (blockIdx.x % 8) * (nall / 8) + blockIdx.x / 8;
+  const uint32_t chunk = logical / nblk;
+  logical -= chunk * nblk;
+  const uint32_t nblocks_n = nblk / mblocks;
+  const uint32_t wm = wave / WN, wn = wave % WN;
+  const uint32_t group = logical / (GM * nblocks_n), first_m = group * GM;
+  const uint32_t gm = mblocks - first_m < GM ? mblocks - first_m : GM;
+  const uint32_t in_group = logical - group * GM * nblocks_n;
+  const uint32_t mb = first_m + in_group % gm, nb = in_group / gm;
+  const uint64_t ksteps = kpad / 128, cper = (ksteps + ks.chunks - 1) / ks.chunks;
+  const uint64_t k0 = uint64_t(chunk) * cper < ksteps ? uint64_t(chunk) * cper : ksteps;
+  const uint64_t nsteps = (k0 + cper < ksteps ? k0 + cper : ksteps) - k0;  // this block's K steps
+  // weight tiles are virtual: digit plane p of tile t is tile t * planes + p
+  // (a block's FB tiles per wave hold whole tiles' planes)
+  const uint64_t ntiles = (n_rows + 15) / 16 << lp;  // (lp = log2 of the digit planes)
   const int planes = 1 << lp;
+  const uint64_t at0 = uint64_t(mb) * TA, bt0 = uint64_t(nb) * TB;
+  // The block's decomposition flags, one vector load per token group (lane p
+  // reads part p's flag, at clamped addresses), issued ahead of the first
+  // step's copies so that waiting for them leaves the copies in flight.
+  const uint64_t parts = limb_parts(kpad);
+  const bool many = parts > kLimbMaxParts;  // (every part of every group takes four limbs)
+  constexpr int NG = TA / 4;                // the block's token groups
+  const uint64_t ngroups = a_tiles / 4;
+  uint32_t flag[NG];
+#pragma unroll
+  for (int t = 0; t < NG; ++t) {
+    const uint64_t grp = at0 / 4 + t < ngroups ? at0 / 4 + t : ngroups - 1;
+    flag[t] = a_flags[grp * parts + (lane < parts ? lane : parts - 1)];
+  }
+  // this wave's copies: chunk c = wave * LPW + u is tile-step c / 2 (A tiles
+  // first), half c % 2; tiles past the matrix re-read its last tile (their
+  // results are never stored); fourth-limb A tiles are not copied in a
+  // three-limb block (the first step copies them before the flags are known)
+  const int8_t* src[LPW];
+  bool limb3[LPW];
+#pragma unroll
+  for (int u = 0; u < LPW; ++u) {
+    const uint32_t c = wave * LPW + u, ts = c >> 1, h = c & 1;
+    const bool is_a = ts < uint32_t(TA);
+    uint64_t tile = is_a ? at0 + ts : (ts < uint32_t(TS) ? bt0 + (ts - TA) : bt0);  // (spare slots: bt0)
+    if (is_a ? tile >= a_tiles : tile >= ntiles) tile = (is_a ? a_tiles : ntiles) - 1;
+    // (weight tile-steps hold each half of the lanes' operands contiguously;
+    // the activation limb tiles keep the 32-byte lane slots)
+    src[u] = (is_a ? a : q) + (tile * ksteps + k0) * 2048 + (is_a ? lane * 32 + h * 16 : h * kTileHalfBytes + lane * 16);
+    limb3[u] = is_a && (ts & 3) == 3;
+  }
+  bool four = true;
+  auto copy_step = [&](uint64_t s, int buf) {
+#pragma unroll
+    for (int u = 0; u < LPW; ++u) {
+      const uint32_t c = wave * LPW + u;
+      if (NBUF > 2 || four || !limb3[u])
+        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(src[u] + s * 2048),
+                                         (void __attribute__((address_space(3)))*)(lds_gemm + (buf * SLOTS + c) * 1024),
+                                         16, 0, 0);
+    }
+  };
+  const v4i zero = {0, 0, 0, 0};
+  v4i acc[FA][FB];
+#pragma unroll
+  for (int i = 0; i < FA; ++i)
+#pragma unroll
+    for (int j = 0; j < FB; ++j) acc[i][j] = zero;
+  // NBUF - 1 steps in flight ahead of the one being multiplied
+#pragma unroll
+  for (int p = 0; p < NBUF - 1; ++p)
+    if (uint64_t(p) < nsteps) copy_step(p, p);
+  // the epilogue's row sums and scales, loaded while the K loop runs
   const uint32_t g = lane >> 4, i = lane & 15;
+  int32_t ep_rowsum[FB], ep_scale[FB];
+#pragma unroll
+  for (int tj = 0; tj < FB; ++tj) {
+    const uint64_t row = ((bt0 + wn * FB + tj) >> lp) * 16 + i;
+    const uint64_t rc = row < n_rows ? row : n_rows - 1;
+    ep_rowsum[tj] = rowsum[rc];
+    ep_scale[tj] = scale[rc];
+  }
+  // per token group, the parts that take four limbs (bit p); the block runs
+  // four limbs when any group needs them anywhere (one limb count for the
+  // whole K range: a loop that switches between the two forms per part needs
+  // more registers than the larger block has)
+  uint64_t gmask[NG];
+  uint64_t fourmask = many ? 1 : 0;
+#pragma unroll
+  for (int t = 0; t < NG; ++t) {
+    const uint64_t bits = __ballot(lane < parts && flag[t] != 0);
+    gmask[t] = !many && at0 / 4 + t < ngroups ? bits : 0;
+    fourmask |= gmask[t];
+  }
+  four = fourmask != 0;
+  // vmcnt immediate: wait until at most (NBUF - 2) steps of copies are outstanding
+  constexpr int kWait = (NBUF - 2) * LPW;
+  static_assert(kWait < 64, "vmcnt range");
+  constexpr int kWaitImm = (kWait & 15) | (7 << 4) | (15 << 8) | ((kWait >> 4) << 14);
+  // Each wave waits for its own copies of a step (vmcnt, in issue order),
+  // then the barrier makes every wave's copies of that step visible. A bare
+  // s_barrier (not __syncthreads, whose fence would wait for every copy in
+  // flight) between compiler memory barriers keeps the later steps' copies
+  // outstanding across it.
+  auto step_barrier = [&](bool more) {
+    asm volatile("" ::: "memory");
+    if (more) __builtin_amdgcn_s_waitcnt(kWaitImm);
+    else __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  step_barrier(nsteps >= uint64_t(NBUF - 1));
+  // the K loop with L limbs (A tiles with i % 4 >= L are neither read nor multiplied)
+  auto kloop = [&](auto Lc) {
+    constexpr int L = decltype(Lc)::value;
+    for (uint64_t s = 0; s < nsteps; ++s) {
+      const int buf = int(s % NBUF);
+      const int8_t* base = lds_gemm + buf * SLOTS * 1024 + lane * 16;
+      // the first half's operands, the copies, the second half's operands
+      // (read while the first half's MFMAs run), then the MFMAs
+      v4i ao[2][FA], bo[2][FB];
+      auto read_half = [&](int h) {
+#pragma unroll
+        for (int j = 0; j < FB; ++j) bo[h][j] = *reinterpret_cast<const v4i*>(base + (TA + wn * FB + j) * 2048 + 1024 * h);
+#pragma unroll
+        for (int i = 0; i < FA; ++i)
+          if ((i & 3) < L) ao[h][i] = *reinterpret_cast<const v4i*>(base + (wm * FA + i) * 2048 + 1024 * h);
+      };
+      read_half(0);
+      if (s + NBUF - 1 < nsteps) copy_step(s + NBUF - 1, int((s + NBUF - 1) % NBUF));
+      read_half(1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < FA; ++i)
+#pragma unroll
+          for (int j = 0; j < FB; ++j)
+            if ((i & 3) < L) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ao[h][i], bo[h][j], acc[i][j], 0, 0, 0);
+      // step s + 1's copies are complete when no more than the later steps' are outstanding
+      step_barrier(s + NBUF - 1 < nsteps);
+    }
+  };
+  if (four) kloop(std::integral_constant<int, 4>());
+  else kloop(std::integral_constant<int, 3>());
   // epilogue: lane 16 g + i holds, in component r of the four limb tiles of a
   // token group, the limb sums of token 16 group + 4 g + r and weight row 16 tile + i
 #pragma unroll
@@ -1503,201 +1680,10 @@ __device__ __forceinline__ void gemm_epilogue(const v4i (&acc)[FA][FB], uint64_t
   }
 }
 
-// Block: TA A tiles (TA / 4 token groups of 16 tokens, four limb tiles each)
-// x TB weight tiles on WM x WN waves, each wave (TA / WM) x (TB / WN) MFMA
-// tiles (whole token groups). A block whose token groups all take three limbs
-// multiplies no fourth-limb tile, and with two buffers does not copy them
-// either (with more, every wave copies a fixed number of tile-step halves per
-// step, so that one vmcnt immediate covers the steps in flight). Every
-// 128-column K step, the block's
-// TA + TB tile-steps (2 KB each) are copied straight from global memory into
-// one of NBUF LDS buffers with global_load_lds_dwordx4 (no register staging).
-// The 2 (TA + TB) copy halves are dealt out LPW per wave; where they do not
-// divide evenly, the slots past them re-copy the block's first weight
-// tile-step half into the buffer's spare kilobytes, so that every wave issues
-// the same copies per step:
-// the copies of the next NBUF - 1 steps are in flight while step s's MFMAs
-// run, and one barrier per step hands a buffer over. Copy h of a tile-step
-// takes the 16-byte half h of every lane's 32 columns (a weight tile-step's
-// contiguous half h; bytes [16 h, 16 h + 16) of each 32-byte slot of an
-// activation tile-step), so each 1 KB LDS half holds one MFMA operand of all
-// 64 lanes contiguously
-// and the 128-bit operand reads do not conflict on LDS banks. The MFMAs of a
-// step run as two passes over the wave's tile pairs (first 64 columns, then
-// the second 64), so consecutive MFMAs never share an accumulator.
-template <int TA, int TB, int WM, int WN, uint32_t GM, int NBUF, bool SPLIT, bool GELU, bool DG>
-__global__ __launch_bounds__(64 * WM * WN) void k_gemm_lds(const int8_t* __restrict__ a, const int8_t* __restrict__ q,
-                                                           const int32_t* __restrict__ scale,
-                                                           const int32_t* __restrict__ rowsum,
-                                                           const int32_t* __restrict__ rowsum_p, uint64_t rowsum_p_ld,
-                                                           uint64_t n_rows, uint64_t kpad, uint64_t m_tokens,
-                                                           uint64_t a_tiles, const uint32_t* __restrict__ a_flags,
-                                                           uint32_t mblocks, int32_t* __restrict__ out,
-                                                           uint64_t ld_out, int64_t* __restrict__ acc_out,
-                                                           RowSplit split, KSplit ks, int lp_arg) {
-  const int lp = DG ? lp_arg : 0;  // (single-plane instances fold it to 0)
-  constexpr int NW = WM * WN;                  // waves
-  constexpr int TS = TA + TB;                  // tile-steps per K step
-  constexpr int LPW = (2 * TS + NW - 1) / NW;  // 1 KB wave copies per wave per K step
-  constexpr int SLOTS = LPW * NW;               // 1 KB copy slots per LDS buffer (>= 2 TS)
-  constexpr int FA = TA / WM, FB = TB / WN;    // MFMA tiles per wave
-  static_assert(FA % 4 == 0 && NBUF >= 2, "whole token groups per wave");
-  extern __shared__ __attribute__((aligned(16))) int8_t lds_gemm[];
-  // the wave index as a scalar, so that copy addresses and LDS targets stay in SGPRs
-  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Block order: block b runs on XCD b % 8, and each XCD takes a contiguous
-  // range of logical blocks; logical blocks go in groups of GM m-blocks x all
-  // n-blocks with m fastest, so the blocks resident on one XCD at a time form
-  // a compact GM x (resident / GM) patch whose A and weight tiles share its L2.
-  // With K split into ks.chunks ranges, chunk c takes logical blocks
-  // [c nblk, (c + 1) nblk) and the same ordering inside them.
-  const uint32_t nall = gridDim.x, nblk = nall / ks.chunks;
-  uint32_t logical = blockIdx.x;
-  if (nall % 8 == 0) logical = (blockIdx.x % 8) * (nall / 8) + blockIdx.x / 8;
-  const uint32_t chunk = logical / nblk;
-  logical -= chunk * nblk;
-  const uint32_t nblocks_n = nblk / mblocks;
-  const uint32_t wm = wave / WN, wn = wave % WN;
-  const uint32_t group = logical / (GM * nblocks_n), first_m = group * GM;
-  const uint32_t gm = mblocks - first_m < GM ? mblocks - first_m : GM;
-  const uint32_t in_group = logical - group * GM * nblocks_n;
-  const uint32_t mb = first_m + in_group % gm, nb = in_group / gm;
-  const uint64_t ksteps = kpad / 128, cper = (ksteps + ks.chunks - 1) / ks.chunks;
-  const uint64_t k0 = uint64_t(chunk) * cper < ksteps ? uint64_t(chunk) * cper : ksteps;
-  const uint64_t nsteps = (k0 + cper < ksteps ? k0 + cper : ksteps) - k0;  // this block's K steps
-  // weight tiles are virtual: digit plane p of tile t is tile t * planes + p
-  // (a block's FB tiles per wave hold whole tiles' planes)
-  const uint64_t ntiles = (n_rows + 15) / 16 << lp;  // (lp = log2 of the digit planes)
-  const uint64_t at0 = uint64_t(mb) * TA, bt0 = uint64_t(nb) * TB;
-  // The block's decomposition flags, one vector load per token group (lane p
-  // reads part p's flag, at clamped addresses), issued ahead of the first
-  // step's copies so that waiting for them leaves the copies in flight.
-  const uint64_t parts = limb_parts(kpad);
-  const bool many = parts > kLimbMaxParts;  // (every part of every group takes four limbs)
-  constexpr int NG = TA / 4;                // the block's token groups
-  const uint64_t ngroups = a_tiles / 4;
-  uint32_t flag[NG];
-#pragma unroll
-  for (int t = 0; t < NG; ++t) {
-    const uint64_t grp = at0 / 4 + t < ngroups ? at0 / 4 + t : ngroups - 1;
-    flag[t] = a_flags[grp * parts + (lane < parts ? lane : parts - 1)];
-  }
-  // this wave's copies: chunk c = wave * LPW + u is tile-step c / 2 (A tiles
-  // first), half c % 2; tiles past the matrix re-read its last tile (their
-  // results are never stored); fourth-limb A tiles are not copied in a
-  // three-limb block (the first step copies them before the flags are known)
-  const int8_t* src[LPW];
-  bool limb3[LPW];
-#pragma unroll
-  for (int u = 0; u < LPW; ++u) {
-    const uint32_t c = wave * LPW + u, ts = c >> 1, h = c & 1;
-    const bool is_a = ts < uint32_t(TA);
-    uint64_t tile = is_a ? at0 + ts : (ts < uint32_t(TS) ? bt0 + (ts - TA) : bt0);  // (spare slots: bt0)
-    if (is_a ? tile >= a_tiles : tile >= ntiles) tile = (is_a ? a_tiles : ntiles) - 1;
-    // (weight tile-steps hold each half of the lanes' operands contiguously;
-    // the activation limb tiles keep the 32-byte lane slots)
-    src[u] = (is_a ? a : q) + (tile * ksteps + k0) * 2048 + (is_a ? lane * 32 + h * 16 : h * kTileHalfBytes + lane * 16);
-    limb3[u] = is_a && (ts & 3) == 3;
-  }
-  bool four = true;
-  auto copy_step = [&](uint64_t s, int buf) {
-#pragma unroll
-    for (int u = 0; u < LPW; ++u) {
-      const uint32_t c = wave * LPW + u;
-      if (NBUF > 2 || four || !limb3[u])
-        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(src[u] + s * 2048),
-                                         (void __attribute__((address_space(3)))*)(lds_gemm + (buf * SLOTS + c) * 1024),
-                                         16, 0, 0);
-    }
-  };
-  const v4i zero = {0, 0, 0, 0};
-  v4i acc[FA][FB];
-#pragma unroll
-  for (int i = 0; i < FA; ++i)
-#pragma unroll
-    for (int j = 0; j < FB; ++j) acc[i][j] = zero;
-  // NBUF - 1 steps in flight ahead of the one being multiplied
-#pragma unroll
-  for (int p = 0; p < NBUF - 1; ++p)
-    if (uint64_t(p) < nsteps) copy_step(p, p);
-  // the epilogue's row sums and scales, loaded while the K loop runs
-  int32_t ep_rowsum[FB], ep_scale[FB];
-#pragma unroll
-  for (int tj = 0; tj < FB; ++tj) {
-    const uint64_t row = ((bt0 + wn * FB + tj) >> lp) * 16 + (lane & 15);
-    const uint64_t rc = row < n_rows ? row : n_rows - 1;
-    ep_rowsum[tj] = rowsum[rc];
-    ep_scale[tj] = scale[rc];
-  }
-  // per token group, the parts that take four limbs (bit p); the block runs
-  // four limbs when any group needs them anywhere (one limb count for the
-  // whole K range: a loop that switches between the two forms per part needs
-  // more registers than the larger block has)
-  uint64_t gmask[NG];
-  uint64_t fourmask = many ? 1 : 0;
-#pragma unroll
-  for (int t = 0; t < NG; ++t) {
-    const uint64_t bits = __ballot(lane < parts && flag[t] != 0);
-    gmask[t] = !many && at0 / 4 + t < ngroups ? bits : 0;
-    fourmask |= gmask[t];
-  }
-  four = fourmask != 0;
-  // vmcnt immediate: wait until at most (NBUF - 2) steps of copies are outstanding
-  constexpr int kWait = (NBUF - 2) * LPW;
-  static_assert(kWait < 64, "vmcnt range");
-  constexpr int kWaitImm = (kWait & 15) | (7 << 4) | (15 << 8) | ((kWait >> 4) << 14);
-  // Each wave waits for its own copies of a step (vmcnt, in issue order),
-  // then the barrier makes every wave's copies of that step visible. A bare
-  // s_barrier (not __syncthreads, whose fence would wait for every copy in
-  // flight) between compiler memory barriers keeps the later steps' copies
-  // outstanding across it.
-  auto step_barrier = [&](bool more) {
-    asm volatile("" ::: "memory");
-    if (more) __builtin_amdgcn_s_waitcnt(kWaitImm);
-    else __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-  step_barrier(nsteps >= uint64_t(NBUF - 1));
-  // the K loop with L limbs (A tiles with i % 4 >= L are neither read nor multiplied)
-  auto kloop = [&](auto Lc) {
-    constexpr int L = decltype(Lc)::value;
-    for (uint64_t s = 0; s < nsteps; ++s) {
-      const int buf = int(s % NBUF);
-      const int8_t* base = lds_gemm + buf * SLOTS * 1024 + lane * 16;
-      // the first half's operands, the copies, the second half's operands
-      // (read while the first half's MFMAs run), then the MFMAs
-      v4i ao[2][FA], bo[2][FB];
-      auto read_half = [&](int h) {
-#pragma unroll
-        for (int j = 0; j < FB; ++j) bo[h][j] = *reinterpret_cast<const v4i*>(base + (TA + wn * FB + j) * 2048 + 1024 * h);
-#pragma unroll
-        for (int i = 0; i < FA; ++i)
-          if ((i & 3) < L) ao[h][i] = *reinterpret_cast<const v4i*>(base + (wm * FA + i) * 2048 + 1024 * h);
-      };
-      read_half(0);
-      if (s + NBUF - 1 < nsteps) copy_step(s + NBUF - 1, int((s + NBUF - 1) % NBUF));
-      read_half(1);
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < FA; ++i)
-#pragma unroll
-          for (int j = 0; j < FB; ++j)
-            if ((i & 3) < L) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ao[h][i], bo[h][j], acc[i][j], 0, 0, 0);
-      // step s + 1's copies are complete when no more than the later steps' are outstanding
-      step_barrier(s + NBUF - 1 < nsteps);
-    }
-  };
-  if (four) kloop(std::integral_constant<int, 4>());
-  else kloop(std::integral_constant<int, 3>());
-  gemm_epilogue<FA, FB, NG, SPLIT, GELU>(acc, at0, bt0, wm, wn, lane, lp, gmask, many, parts, chunk, ep_rowsum, ep_scale,
-                                         rowsum_p, rowsum_p_ld, n_rows, m_tokens, out, ld_out, acc_out, split, ks);
-}
-
-// The same tiles and epilogue as k_gemm_lds on few large waves: the K range in
-// 64-column stages (half a tile-step, 1 KB per tile) through a ring of NBUF
-// LDS buffers, the operands of the next stage read from LDS into a second
+// The gate/up GELU product of two-plane weights (W as for k_gemm_lds's GELU
+// form) on few large waves: 64 tokens x 64 rows (128 virtual) on 4 waves, the K
+// range in 64-column stages (half a tile-step, 1 KB per tile) through a ring of
+// three LDS buffers, the operands of the next stage read from LDS into a second
 // register set while this stage's MFMAs run. A stage's copies are dealt out
 // LPW per wave, the three-limb A tiles and the weights first and the
 // fourth-limb tiles last, so that only the last wave's count depends on the
@@ -1705,64 +1691,63 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_lds(const int8_t* __restr
 // flags are known. What bounds it is what bounds k_gemm_lds: int8 MFMAs alone
 // run at 3.0 POP/s on random limbs (the clock drops under them), both kernels
 // reach 1.8-2.0, and for plain outputs k_gemm_lds is as fast or faster at
-// every shape (20480 x 2560 at 2048 rows 342 against 355 us). It serves the
-// gate/up GELU product of two-plane weights, whose larger wave tiles and two
-// blocks per CU beat the 128 x 128 blocks: a sliding and a full E4B-width layer
-// of i16 weights 2785 -> 2613 us at 1643 rows, 1465 -> 1394 at 800, 661 -> 641
-// at 200. (Single planes have twice the epilogue per product and keep the
+// every shape (20480 x 2560 at 2048 rows 342 against 355 us). Here the larger
+// wave tiles and two blocks per CU beat the 128 x 128 blocks: a sliding and a
+// full E4B-width layer of i16 weights 2785 -> 2613 us at 1643 rows, 1465 ->
+// 1394 at 800. (Single planes have twice the epilogue per product and keep the
 // finer blocks: 1890 against 1972 us.)
-template <int TA, int TB, int WM, int WN, uint32_t GM, int NBUF, bool SPLIT, bool GELU, bool DG>
-__global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_ring(
+constexpr int kRingTA = 16, kRingTB = 8, kRingBufs = 3;  // A and weight tiles per block, LDS buffers
+__global__ __launch_bounds__(256, 2) void k_gemm_ring_gelu(
     const int8_t* __restrict__ a, const int8_t* __restrict__ q, const int32_t* __restrict__ scale,
     const int32_t* __restrict__ rowsum, const int32_t* __restrict__ rowsum_p, uint64_t rowsum_p_ld, uint64_t n_rows,
     uint64_t kpad, uint64_t m_tokens, uint64_t a_tiles, const uint32_t* __restrict__ a_flags, uint32_t mblocks,
-    int32_t* __restrict__ out, uint64_t ld_out, int64_t* __restrict__ acc_out, RowSplit split, KSplit ks, int lp_arg) {
-  const int lp = DG ? lp_arg : 0;  // (single-plane instances fold it to 0)
-  constexpr int NW = WM * WN;
-  constexpr int NG = TA / 4;                 // the block's token groups
+    int32_t* __restrict__ out, uint64_t ld_out) {
+  constexpr int TA = kRingTA, TB = kRingTB, NBUF = kRingBufs, WN = 2, NW = 4;
+  constexpr uint32_t GM = 4;                  // m-blocks per group of the block order
+  constexpr int NG = TA / 4;                  // the block's token groups
   constexpr int TS = TA + TB, LPW = TS / NW;  // 1 KB copies per stage, per wave
-  constexpr int FA = TA / WM, FB = TB / WN;  // MFMA tiles per wave
+  constexpr int FA = TA / 2, FB = TB / WN;    // MFMA tiles per wave
   static_assert(TS % NW == 0 && NG <= LPW && FA % 4 == 0, "whole shares; the fourth limbs in the last wave's");
   extern __shared__ __attribute__((aligned(16))) int8_t lds_gemm[];
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // block order as in k_gemm_lds
-  const uint32_t nall = gridDim.x, nblk = nall / ks.chunks;
+  const uint32_t nall = gridDim.x;
   uint32_t logical = blockIdx.x;
   if (nall % 8 == 0) logical = (blockIdx.x % 8) * (nall / 8) + blockIdx.x / 8;
-  const uint32_t chunk = logical / nblk;
-  logical -= chunk * nblk;
-  const uint32_t nblocks_n = nblk / mblocks;
+  const uint32_t nblocks_n = nall / mblocks;
   const uint32_t wm = wave / WN, wn = wave % WN;
   const uint32_t group = logical / (GM * nblocks_n), first_m = group * GM;
   const uint32_t gm = mblocks - first_m < GM ? mblocks - first_m : GM;
   const uint32_t in_group = logical - group * GM * nblocks_n;
   const uint32_t mb = first_m + in_group % gm, nb = in_group / gm;
-  const uint64_t ksteps = kpad / 128, cper = (ksteps + ks.chunks - 1) / ks.chunks;
-  const uint64_t k0 = uint64_t(chunk) * cper < ksteps ? uint64_t(chunk) * cper : ksteps;
-  const uint32_t nst = 2 * uint32_t((k0 + cper < ksteps ? k0 + cper : ksteps) - k0);  // this block's stages
-  const uint64_t ntiles = (n_rows + 15) / 16 << lp;
+  const uint64_t ksteps = kpad / 128;
+  const uint32_t nst = 2 * uint32_t(ksteps);  // stages
+  const uint64_t ntiles = (n_rows + 15) / 16 * 2;  // virtual tiles: tile t's planes are 2 t and 2 t + 1
   const uint64_t at0 = uint64_t(mb) * TA, bt0 = uint64_t(nb) * TB;
   const uint64_t parts = limb_parts(kpad);
   const bool many = parts > kLimbMaxParts;
   const uint64_t ngroups = a_tiles / 4;
+  // the block's decomposition flags (as in k_gemm_lds) and the epilogue's row
+  // sums and scales, ahead of the copies: they come back first
   uint32_t flag[NG];
 #pragma unroll
   for (int t = 0; t < NG; ++t) {
     const uint64_t grp = at0 / 4 + t < ngroups ? at0 / 4 + t : ngroups - 1;
     flag[t] = a_flags[grp * parts + (lane < parts ? lane : parts - 1)];
   }
-  // (the epilogue's row sums and scales, ahead of the copies for the same reason)
-  int32_t ep_rowsum[FB], ep_scale[FB];
+  int32_t ep_rowsum[FB / 2], ep_scale[FB / 2];
 #pragma unroll
-  for (int tj = 0; tj < FB; ++tj) {
-    const uint64_t row = ((bt0 + wn * FB + tj) >> lp) * 16 + (lane & 15);
+  for (int tj = 0; tj < FB / 2; ++tj) {
+    const uint64_t row = ((bt0 + wn * FB) / 2 + tj) * 16 + (lane & 15);
     const uint64_t rc = row < n_rows ? row : n_rows - 1;
     ep_rowsum[tj] = rowsum[rc];
     ep_scale[tj] = scale[rc];
   }
   // slot c of a stage: A tiles of limbs 0-2 (group c / 3), then the weight
   // tiles, then the groups' fourth limbs; LDS position `pos` (A tile 4 g + j,
-  // or TA + weight tile). Tiles past the matrix re-read its last tile.
+  // or TA + weight tile). Tiles past the matrix re-read its last tile. The
+  // sources are wave-uniform; lane offsets: 16 bytes in a weight tile-step's
+  // contiguous half, 32 in an activation tile-step.
   const int8_t* src[LPW];
   uint32_t pos[LPW];
 #pragma unroll
@@ -1772,7 +1757,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_ring(
     pos[u] = c < 3 * NG ? 4 * (c / 3) + c % 3 : (is_b ? TA + (c - 3 * NG) : 4 * (c - 3 * NG - TB) + 3);
     uint64_t tile = is_b ? bt0 + (pos[u] - TA) : at0 + pos[u];
     if (tile >= (is_b ? ntiles : a_tiles)) tile = (is_b ? ntiles : a_tiles) - 1;
-    src[u] = (is_b ? q : a) + (tile * ksteps + k0) * 2048 + (is_b ? lane * 16 : lane * 32);
+    src[u] = (is_b ? q : a) + tile * ksteps * 2048;
   }
   const bool last = wave == NW - 1;
   // stage s, its three-limb slots (part 1) and / or its fourth-limb slots (part 2)
@@ -1783,9 +1768,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_ring(
       const uint32_t c = wave * LPW + u;
       const bool fourth = c >= uint32_t(3 * NG + TB), is_b = pos[u] >= uint32_t(TA);
       if (parts12 & (fourth ? 2 : 1))
-        __builtin_amdgcn_global_load_lds(
-            (const void __attribute__((address_space(1)))*)(src[u] + uint64_t(s >> 1) * 2048 + (s & 1) * (is_b ? 1024 : 16)),
-            (void __attribute__((address_space(3)))*)(buf + pos[u] * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(
+                                             src[u] + (uint64_t(s >> 1) * 2048 + (s & 1) * (is_b ? 1024 : 16)) +
+                                             (is_b ? lane * 16 : lane * 32)),
+                                         (void __attribute__((address_space(3)))*)(buf + pos[u] * 1024), 16, 0, 0);
     }
   };
 #pragma unroll
@@ -1844,16 +1830,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_ring(
     // (with four limbs the first stages' copies are not in stage order)
     stage_barrier(!four && nst >= uint32_t(NBUF));
     read_stage(0, ao[0], bo[0]);
-    // stage s's operands are in set s & 1; nst is even
+    // stage s's operands are in set s & 1 with three limbs (nst is even); with
+    // four, whose two sets would not fit the registers, one set is read again
+    // once the products have taken it
     auto half = [&](uint32_t s, int set) {
+      const int cur = L == 3 ? set : 0, next = L == 3 ? set ^ 1 : 0;
+      if (L == 4) multiply(ao[cur], bo[cur]);
       if (s + 1 < nst) {
         // every wave has read stage s, whose buffer takes stage s + NBUF, and
         // stage s + 1's copies are complete
         stage_barrier(s + NBUF - 1 < nst);
         if (s + NBUF < nst) copy_stage(s + NBUF, four ? 3 : 1);
-        read_stage(s + 1, ao[set ^ 1], bo[set ^ 1]);
+        read_stage(s + 1, ao[next], bo[next]);
       }
-      multiply(ao[set], bo[set]);
+      if (L == 3) multiply(ao[cur], bo[cur]);
     };
     for (uint32_t s = 0; s < nst; s += 2) {
       half(s, 0);
@@ -1862,8 +1852,58 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_ring(
   };
   if (four) kloop(std::integral_constant<int, 4>());
   else kloop(std::integral_constant<int, 3>());
-  gemm_epilogue<FA, FB, NG, SPLIT, GELU>(acc, at0, bt0, wm, wn, lane, lp, gmask, many, parts, chunk, ep_rowsum, ep_scale,
-                                         rowsum_p, rowsum_p_ld, n_rows, m_tokens, out, ld_out, acc_out, split, ks);
+  // (the sums as 32-bit registers here: else their widening moves into the two
+  // loops and the pairs do not fit)
+#pragma unroll
+  for (int i = 0; i < FA; ++i)
+#pragma unroll
+    for (int j = 0; j < FB; ++j) asm volatile("" : "+v"(acc[i][j]));
+  // epilogue: the layout and the arithmetic of k_gemm_lds's GELU form; a real
+  // tile's two planes are consecutive virtual tiles of the wave
+  const uint32_t g = lane >> 4, i = lane & 15;
+#pragma unroll
+  for (int tg = 0; tg < FA / 4; ++tg) {
+    const uint64_t grp = (at0 + wm * FA) / 4 + tg;
+    uint64_t wmask = 0;  // this group's four-limb parts
+#pragma unroll
+    for (int t = 0; t < NG; ++t)
+      if (uint32_t(t) == wm * (FA / 4) + tg) wmask = gmask[t];
+#pragma unroll
+    for (int tj = 0; tj < FB / 2; ++tj) {
+      const uint64_t tile = (bt0 + wn * FB) / 2 + tj, row = tile * 16 + i;
+      const uint64_t rc = row < n_rows ? row : n_rows - 1;
+      const bool all4 = many || wmask == (parts >= 64 ? ~uint64_t(0) : (uint64_t(1) << parts) - 1);
+      uint64_t cterm = uint64_t(int64_t(all4 ? 8421504 : 32896) * ep_rowsum[tj]);
+      if (!all4)
+        for (uint64_t gm4 = wmask; gm4; gm4 &= gm4 - 1)
+          cterm += uint64_t(int64_t(8388608) * rowsum_p[uint64_t(__builtin_ctzll(gm4)) * rowsum_p_ld + rc]);
+      int32_t val[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        uint64_t dot = cterm;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const v4i &d0 = acc[4 * tg][2 * tj + p], &d1 = acc[4 * tg + 1][2 * tj + p], &d2 = acc[4 * tg + 2][2 * tj + p],
+                    &d3 = acc[4 * tg + 3][2 * tj + p];
+          const int64_t d =
+              int64_t(d0[r]) + int64_t(d1[r]) * 256 + int64_t(d2[r]) * 65536 + int64_t(d3[r]) * 16777216;
+          dot += uint64_t(d) << (8 * p);
+        }
+        val[r] = requant(int64_t(dot * uint64_t(int64_t(ep_scale[tj]))));
+      }
+      const bool lo = i < 8;
+      const int32_t send0 = lo ? val[2] : val[0], send1 = lo ? val[3] : val[1];
+      const int32_t recv0 = __shfl(send0, int(lane ^ 8u), 64), recv1 = __shfl(send1, int(lane ^ 8u), 64);
+      const int32_t g0 = lo ? val[0] : recv0, u0 = lo ? recv0 : val[2];
+      const int32_t g1 = lo ? val[1] : recv1, u1 = lo ? recv1 : val[3];
+      const uint64_t f = tile * 8 + (i & 7);
+      const uint64_t t0 = grp * 16 + 4 * g + (lo ? 0 : 2);
+      if (row < n_rows) {  // (whole tiles: the up row is there too)
+        if (t0 < m_tokens) out[t0 * ld_out + f] = mul_sat(gelu_act(g0), u0);
+        if (t0 + 1 < m_tokens) out[(t0 + 1) * ld_out + f] = mul_sat(gelu_act(g1), u1);
+      }
+    }
+  }
 }
 
 // Sum of the K-range planes of a split GEMM (wrapping, so exactly the
@@ -3071,21 +3111,18 @@ static void launch_gemm_lds_dg(const DevMatrix& W, uint64_t m, int32_t* out, uin
                      uint32_t(mblocks), out, ld_out, acc_out, split, ks, plane_log2(W));
 }
 
-template <int TA, int TB, int WM, int WN, uint32_t GM, int NBUF, bool SPLIT, bool GELU, bool DG>
-static void launch_gemm_ring_dg(const DevMatrix& W, uint64_t m, int32_t* out, uint64_t ld_out, int64_t* acc_out,
-                                const int8_t* a_tiled, uint64_t a_tiles, hipStream_t s, RowSplit split) {
-  constexpr uint32_t lds = uint32_t(NBUF) * uint32_t(TA + TB) * 1024u;
+static void launch_gemm_ring_gelu(const DevMatrix& W, uint64_t m, int32_t* out, uint64_t ld_out, const int8_t* a_tiled,
+                                  uint64_t a_tiles, hipStream_t s) {
+  constexpr uint32_t lds = uint32_t(kRingBufs) * uint32_t(kRingTA + kRingTB) * 1024u;
   static_assert(lds <= 160u * 1024u, "LDS of one workgroup");
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&k_gemm_ring<TA, TB, WM, WN, GM, NBUF, SPLIT, GELU, DG>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_ring_gelu),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
   (void)attr;
-  const uint64_t mblocks = (m + 4 * TA - 1) / (4 * TA);
-  const uint64_t nblocks = ((W.rows + 15) / 16 * uint64_t(W.planes) + TB - 1) / TB;
-  hipLaunchKernelGGL((k_gemm_ring<TA, TB, WM, WN, GM, NBUF, SPLIT, GELU, DG>), dim3(unsigned(mblocks * nblocks)),
-                     dim3(64 * WM * WN), lds, s, a_tiled, W.q, W.scale, W.rowsum, W.rowsum_p, W.rowsum_p_ld, W.rows,
-                     W.kpad, m, a_tiles, gemm_flags(a_tiled, m, W.kpad), uint32_t(mblocks), out, ld_out, acc_out, split,
-                     KSplit{}, plane_log2(W));
+  const uint64_t mblocks = (m + 4 * kRingTA - 1) / (4 * kRingTA);
+  const uint64_t nblocks = ((W.rows + 15) / 16 * 2 + kRingTB - 1) / kRingTB;
+  hipLaunchKernelGGL(k_gemm_ring_gelu, dim3(unsigned(mblocks * nblocks)), dim3(256), lds, s, a_tiled, W.q, W.scale,
+                     W.rowsum, W.rowsum_p, W.rowsum_p_ld, W.rows, W.kpad, m, a_tiles, gemm_flags(a_tiled, m, W.kpad),
+                     uint32_t(mblocks), out, ld_out);
 }
 template <int TA, int TB, int WM, int WN, uint32_t GM, int NBUF, bool SPLIT = false, bool GELU = false>
 static void launch_gemm_lds_shape(const DevMatrix& W, uint64_t m, int32_t* out, uint64_t ld_out, int64_t* acc_out,
@@ -3284,10 +3321,10 @@ void launch_gemm_tiled_gelu(const DevMatrix& W, uint64_t m, int32_t* out, uint64
   const PadShape pad = gemm_pad_shape(W, m);
   if (pad != PadShape::kNone)
     return launch_gemm_pad<false, true>(pad, W, m, out, ld_out, nullptr, a_tiled, a_tiles, s, {});
-  // two digit planes past 128 rows: 64 tokens x 128 rows on 4 large waves
-  // (figures at k_gemm_ring)
+  // two digit planes past 128 rows: 64 tokens x 64 rows on 4 large waves
+  // (figures at k_gemm_ring_gelu)
   if (W.planes == 2 && m > 128)
-    return launch_gemm_ring_dg<16, 8, 2, 2, 4, 3, false, true, true>(W, m, out, ld_out, nullptr, a_tiled, a_tiles, s, {});
+    return launch_gemm_ring_gelu(W, m, out, ld_out, a_tiled, a_tiles, s);
   launch_gemm_lds_shape<8, 8, 2, 4, 8, 2, false, true>(W, m, out, ld_out, nullptr, a_tiled, a_tiles, s);
 }
 

@@ -154,6 +154,28 @@ def test_i16_e4b_shaped_capture_matches_oracle(i16_two_layers, prompt_len):
     assert got["end_to_end"] == exp["end_to_end"]
 
 
+@pytest.mark.parametrize("gain,prompt_len", [(60, 193), (4000, 130), (1, 129)])
+def test_i16_gelu_large_wave_blocks_with_four_limbs(ctx, gain, prompt_len):
+    """The large-wave gate/up product past 128 rows: a pre-FF norm gain that takes one column past 24 bits for
+    about one token in thirty (blocks and token groups of three and of four limbs side by side) or for nearly
+    every token, a last block of one weight tile, and a last token group of one or two rows."""
+    cfg = synthetic.e4b_config(layers=2, vocab=512, sliding_window=64)
+    cfg["text_config"].update({"hidden_size": 320, "intermediate_size": 1032, "head_dim": 64,
+                               "num_attention_heads": 4, "num_key_value_heads": 2})
+    tensors = []
+    for name, v, s in synthetic.synthetic_model_i16(cfg, seed=gain):
+        if "pre_feedforward_layernorm" in name:
+            v = v.copy()
+            v[100] = gain << 16
+        tensors.append((name, v, s))
+    om, gm = fixtures.load_both(cfg, tensors, ctx, threads=THREADS)
+    assert gm.fused_decode  # (its interleaved gate/up matrix is what the product reads)
+    prompt = np.random.default_rng(prompt_len).integers(0, 512, size=prompt_len).tolist()
+    exp, got = om.capture(prompt, 2), gm.capture(prompt, 2)
+    assert got["prefill"] == exp["prefill"]
+    assert got["decode_steps"] == exp["decode_steps"]
+
+
 @pytest.mark.parametrize("n", [3, 16])
 def test_i16_e4b_shaped_batch_matches_solo(i16_two_layers, n):
     # batched fused steps (4-token and 16-token GEMVs over the digit planes)
