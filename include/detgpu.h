@@ -70,7 +70,8 @@ void det_event_destroy(det_event_t* ev);
    not run; only calls that allocate nothing and do not synchronize may be
    recorded (run each once beforehand so that their scratch exists; a call
    whose scratch would grow is refused), and the buffers they name must
-   outlive the graph. A failed or refused call ends the capture and discards
+   outlive the graph (scratch that the context or a det_scratch replaces with
+   a larger one later stays allocated as long as the graph). A failed or refused call ends the capture and discards
    what was recorded; det_ctx_capture_end then reports that no capture is in
    progress. */
 int det_ctx_capture_begin(det_ctx_t* ctx);

@@ -51,26 +51,41 @@ thread_local std::string g_error;  // errors before a context exists
 
 }  // namespace
 
+// Device memory with shared ownership: a recorded graph keeps the scratch it
+// uses past the scratch's replacement or its owner's end.
+using DevRef = std::shared_ptr<void>;
+static DevRef dev_alloc(size_t bytes) {
+  void* p = nullptr;
+  HIPC(hipMalloc(&p, bytes));
+  return DevRef(p, [](void* q) { (void)hipFree(q); });
+}
+// One scratch buffer that grows on demand.
+template <class T>
+struct Scratch {
+  DevRef mem;
+  size_t bytes = 0;
+  T* get() const { return static_cast<T*>(mem.get()); }
+  void drop() {
+    mem.reset();
+    bytes = 0;
+  }
+};
+
 struct det_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   int64_t* noalloc_parts = nullptr;  // this device's address of the allocation-free argmax scratch
   std::string last_error;
-  int8_t* limbs = nullptr;  // activation limb scratch for the int8 GEMV
-  size_t limbs_bytes = 0;
-  int64_t* argmax_scratch = nullptr;
-  size_t argmax_parts = 0;
+  Scratch<int8_t> limbs;  // activation limb scratch for the int8 GEMV
+  Scratch<int64_t> argmax_parts;
   uint32_t* argmax_out = nullptr;
 
-  int8_t* gemm_a = nullptr;  // tiled activation limb rows for the prefill GEMM
-  size_t gemm_a_bytes = 0;
-  int64_t* gemm_planes = nullptr;  // K-range partial planes of split GEMMs
-  size_t gemm_planes_bytes = 0;
-  void* attn_work = nullptr;  // work area of the MFMA form of causal attention
-  size_t attn_work_bytes = 0;
-  void* rows_work = nullptr;  // activation rows of a session's prefill (PrefillRows)
-  size_t rows_work_bytes = 0;
-  bool capturing = false;  // between det_ctx_capture_begin and _end
+  Scratch<int8_t> gemm_a;        // tiled activation limb rows for the prefill GEMM
+  Scratch<int64_t> gemm_planes;  // K-range partial planes of split GEMMs
+  Scratch<void> attn_work;       // work area of the MFMA form of causal attention
+  Scratch<void> rows_work;       // activation rows of a session's prefill (PrefillRows)
+  bool capturing = false;        // between det_ctx_capture_begin and _end
+  std::vector<DevRef> recorded;  // scratch objects of the calls recorded since then
 
   // scratch that has to grow cannot be allocated while the stream records
   void grow_check(const char* what) const {
@@ -78,28 +93,22 @@ struct det_ctx {
       bail(std::string("det_ctx capture: ") + what +
            " scratch would grow inside the capture; run the call once before capturing");
   }
-  void ensure_gemm_a(size_t bytes) {
-    if (bytes <= gemm_a_bytes) return;
-    grow_check("GEMM activation");
+  template <class T>
+  void grow(Scratch<T>& b, size_t bytes, const char* what) {
+    if (bytes <= b.bytes) return;
+    grow_check(what);
     HIPC(hipStreamSynchronize(stream));
-    if (gemm_a) HIPC(hipFree(gemm_a));
-    gemm_a = nullptr;
-    HIPC(hipMalloc(&gemm_a, bytes));
-    gemm_a_bytes = bytes;
+    b.drop();
+    b.mem = dev_alloc(bytes);
+    b.bytes = bytes;
   }
+  void ensure_gemm_a(size_t bytes) { grow(gemm_a, bytes, "GEMM activation"); }
   // the partial planes a GEMM of W over m rows splits K into (null: no split)
   int64_t* gemm_planes_for(const det::DevMatrix& W, uint64_t m) {
     const size_t bytes = det::gemm_plane_bytes(W, m);
     if (bytes == 0) return nullptr;
-    if (bytes > gemm_planes_bytes) {
-      grow_check("GEMM partial-plane");
-      HIPC(hipStreamSynchronize(stream));
-      if (gemm_planes) HIPC(hipFree(gemm_planes));
-      gemm_planes = nullptr;
-      HIPC(hipMalloc(&gemm_planes, bytes));
-      gemm_planes_bytes = bytes;
-    }
-    return gemm_planes;
+    grow(gemm_planes, bytes, "GEMM partial-plane");
+    return gemm_planes.get();
   }
   // The MFMA attention's work area for a (null where that form does not
   // apply or would need more than kAttnWorkMax bytes even in query chunks: the
@@ -111,28 +120,12 @@ struct det_ctx {
     a.work = nullptr;
     a.work_bytes = 0;
     if (bytes == 0 || bytes > kAttnWorkMax) return;
-    if (bytes > attn_work_bytes) {
-      if (capturing && det::attn_mfma_unchunked_bytes(a) > kAttnWorkMax) return;
-      grow_check("attention");
-      HIPC(hipStreamSynchronize(stream));
-      if (attn_work) HIPC(hipFree(attn_work));
-      attn_work = nullptr;
-      HIPC(hipMalloc(&attn_work, bytes));
-      attn_work_bytes = bytes;
-    }
-    a.work = attn_work;
-    a.work_bytes = attn_work_bytes;
+    if (bytes > attn_work.bytes && capturing && det::attn_mfma_unchunked_bytes(a) > kAttnWorkMax) return;
+    grow(attn_work, bytes, "attention");
+    a.work = attn_work.get();
+    a.work_bytes = attn_work.bytes;
   }
-  void ensure_rows_work(size_t bytes) {
-    if (bytes <= rows_work_bytes) return;
-    grow_check("prefill row");
-    HIPC(hipStreamSynchronize(stream));
-    if (rows_work) HIPC(hipFree(rows_work));
-    rows_work = nullptr;
-    rows_work_bytes = 0;
-    HIPC(hipMalloc(&rows_work, bytes));
-    rows_work_bytes = bytes;
-  }
+  void ensure_rows_work(size_t bytes) { grow(rows_work, bytes, "prefill row"); }
   // Slab GEMM / GEMV dispatch: int8 weights with at least kGemmMinRows
   // activation rows take the MFMA GEMM, everything else the GEMV kernels.
   static constexpr uint64_t kGemmMinRows = 16;
@@ -141,9 +134,9 @@ struct det_ctx {
     if (W.storage == det::kInt8 && m >= kGemmMinRows) {
       ensure_gemm_a(det::gemm_act_bytes(m, W.kpad));
       int64_t* planes = gemm_planes_for(W, m);
-      det::launch_gemm(W, act, m, ld_act, out, ld_out, acc_out, gemm_a, stream, planes);
+      det::launch_gemm(W, act, m, ld_act, out, ld_out, acc_out, gemm_a.get(), stream, planes);
     } else {
-      det::launch_linear(W, act, m, ld_act, out, ld_out, acc_out, limbs, stream);
+      det::launch_linear(W, act, m, ld_act, out, ld_out, acc_out, limbs.get(), stream);
     }
   }
 
@@ -160,33 +153,18 @@ struct det_ctx {
       return;
     }
     ensure_gemm_a(det::gemm_act_bytes(m, first->kpad));
-    det::launch_gemm_limbs(act, m, first->cols, ld_act, first->kpad, gemm_a, stream);
+    det::launch_gemm_limbs(act, m, first->cols, ld_act, first->kpad, gemm_a.get(), stream);
     for (const auto& it : items) {
       int64_t* planes = gemm_planes_for(*it.first, m);
-      det::launch_gemm_tiled(*it.first, m, it.second, it.first->rows, nullptr, gemm_a, stream, nullptr, planes);
+      det::launch_gemm_tiled(*it.first, m, it.second, it.first->rows, nullptr, gemm_a.get(), stream, nullptr, planes);
     }
   }
 
-  void ensure_limbs(size_t bytes) {
-    if (bytes <= limbs_bytes) return;
-    grow_check("GEMV limb");
-    HIPC(hipStreamSynchronize(stream));
-    if (limbs) HIPC(hipFree(limbs));
-    limbs = nullptr;
-    HIPC(hipMalloc(&limbs, bytes));
-    limbs_bytes = bytes;
-  }
+  void ensure_limbs(size_t bytes) { grow(limbs, bytes, "GEMV limb"); }
   uint32_t argmax(const int32_t* x, uint64_t n) {
     if (capturing) bail("det_ctx capture: the argmax returns its index to the host and cannot be recorded");
-    const size_t parts = (n + 1023) / 1024;
-    if (parts > argmax_parts) {
-      HIPC(hipStreamSynchronize(stream));
-      if (argmax_scratch) HIPC(hipFree(argmax_scratch));
-      argmax_scratch = nullptr;
-      HIPC(hipMalloc(&argmax_scratch, parts * sizeof(int64_t)));
-      argmax_parts = parts;
-    }
-    det::launch_argmax(x, n, argmax_scratch, argmax_out, stream);
+    grow(argmax_parts, (n + 1023) / 1024 * sizeof(int64_t), "argmax");
+    det::launch_argmax(x, n, argmax_parts.get(), argmax_out, stream);
     uint32_t r = 0;
     HIPC(hipMemcpyAsync(&r, argmax_out, 4, hipMemcpyDeviceToHost, stream));
     HIPC(hipStreamSynchronize(stream));
@@ -205,6 +183,7 @@ struct det_event {
 struct det_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  std::vector<DevRef> scratch;  // what the recorded calls use besides their arguments
   ~det_graph() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -218,6 +197,7 @@ namespace {
 void abort_capture(det_ctx* ctx) {
   if (!ctx || !ctx->capturing) return;
   ctx->capturing = false;
+  ctx->recorded.clear();
   hipGraph_t g = nullptr;
   (void)hipStreamEndCapture(ctx->stream, &g);
   if (g) (void)hipGraphDestroy(g);
@@ -1100,10 +1080,10 @@ struct det_kv {
 struct det_scratch {
   det_model* m = nullptr;
   det_ctx* ctx = nullptr;  // m->ctx, kept so that freeing the scratch does not read the model
-  std::unique_ptr<det_session> ws;
+  std::shared_ptr<det_session> ws;
   // the fused step's buffers for det_layer_decode, for caches of up to
   // dec->score_stride rows
-  std::unique_ptr<det_session> dec;
+  std::shared_ptr<det_session> dec;
 };
 
 namespace {
@@ -1217,7 +1197,7 @@ struct PrefillRows {
     });
     ses->ctx->ensure_rows_work(bytes);
     bytes = 0;
-    uint8_t* base = static_cast<uint8_t*>(ses->ctx->rows_work);
+    uint8_t* base = static_cast<uint8_t*>(ses->ctx->rows_work.get());
     row_buffers(ses, n, [&](uint64_t b) -> void* { return base + slot(b); });
     s = ses;
   }
@@ -1230,11 +1210,9 @@ struct PrefillRows {
     s->vb = own.vb, s->attn = own.attn, s->gate = own.gate, s->up = own.up, s->ple_all = own.ple_all;
     s->pe = own.pe, s->pp = own.pp;
     det_ctx* ctx = s->ctx;
-    if (ctx->rows_work_bytes > kRowsWorkMax) {
+    if (ctx->rows_work.bytes > kRowsWorkMax) {
       (void)hipStreamSynchronize(ctx->stream);
-      (void)hipFree(ctx->rows_work);
-      ctx->rows_work = nullptr;
-      ctx->rows_work_bytes = 0;
+      ctx->rows_work.drop();
     }
   }
 };
@@ -1396,14 +1374,14 @@ bool qkv_block(det_session* s, const GLayer& L, uint64_t M, uint64_t pos0, const
   if (L.v && QKV && M >= det_ctx::kGemmMinRows && QKV->storage == det::kInt8 && QKV->planes <= 2 && QKV->rows == qw + 2 * kw &&
       L.q->rows == qw && L.k->rows == kw && L.v->rows == kw && qw % 16 == 0 && kw % 16 == 0) {
     ctx->ensure_gemm_a(det::gemm_act_bytes(M, QKV->kpad));
-    det::launch_gemm_limbs(s->normed, M, QKV->cols, L.q->cols, QKV->kpad, ctx->gemm_a, st);
+    det::launch_gemm_limbs(s->normed, M, QKV->cols, L.q->cols, QKV->kpad, ctx->gemm_a.get(), st);
     det::RowSplit sp;
     sp.out1 = s->kb;
     sp.out2 = s->vb;
     sp.ld1 = sp.ld2 = kw;
     sp.r1 = qw;
     sp.r2 = qw + kw;
-    det::launch_gemm_tiled(*QKV, M, s->qb, qw, nullptr, ctx->gemm_a, st, &sp, ctx->gemm_planes_for(*QKV, M));
+    det::launch_gemm_tiled(*QKV, M, s->qb, qw, nullptr, ctx->gemm_a.get(), st, &sp, ctx->gemm_planes_for(*QKV, M));
   } else if (L.v) {
     ctx->linear_group({{L.q, s->qb}, {L.k, s->kb}, {L.v, s->vb}}, s->normed, M, L.q->cols);
   } else if (L.k_eq_v) {
@@ -1483,8 +1461,8 @@ bool post_attention(det_session* s, const GLayer& L, uint64_t M, const int32_t* 
   if (GU && M >= det_ctx::kGemmMinRows && GU->storage == det::kInt8 && GU->planes <= 2 && GU->rows == 2 * L.gate->rows &&
       GU->cols == H && L.gate->rows % 8 == 0) {
     ctx->ensure_gemm_a(det::gemm_act_bytes(M, GU->kpad));
-    det::launch_gemm_limbs(s->normed, M, H, H, GU->kpad, ctx->gemm_a, st);
-    det::launch_gemm_tiled_gelu(*GU, M, s->gate, L.gate->rows, ctx->gemm_a, st);
+    det::launch_gemm_limbs(s->normed, M, H, H, GU->kpad, ctx->gemm_a.get(), st);
+    det::launch_gemm_tiled_gelu(*GU, M, s->gate, L.gate->rows, ctx->gemm_a.get(), st);
   } else {
     ctx->linear_group({{L.gate, s->gate}, {L.up, s->up}}, s->normed, M, H);
     det::launch_gelu_mul(s->gate, s->up, M * L.gate->rows, st);
@@ -3094,12 +3072,13 @@ bool trace_run(det_model* m, const det_trace_request_t* rq, TraceCollector& tc) 
 det_session* scratch_rows(det_scratch* sc, uint64_t rows) {
   if (!sc->ws || sc->ws->max_tokens < rows) {
     HIPC(hipStreamSynchronize(sc->m->ctx->stream));
-    auto w = std::make_unique<det_session>();
+    auto w = std::make_shared<det_session>();
     w->m = sc->m;
     w->max_tokens = std::max<uint64_t>(rows, sc->ws ? 2 * sc->ws->max_tokens : 16);
     session_alloc(w.get(), false);
     sc->ws = std::move(w);
   }
+  if (sc->m->ctx->capturing) sc->m->ctx->recorded.push_back(sc->ws);
   return sc->ws.get();
 }
 
@@ -3129,7 +3108,7 @@ bool layer_decode_fused(det_scratch* sc, uint64_t l, const int32_t* input, const
   if (!sc->dec || sc->dec->score_stride < ac.cap) {
     if (ctx->capturing) return false;  // (no allocation while the stream records)
     HIPC(hipStreamSynchronize(st));
-    auto w = std::make_unique<det_session>();
+    auto w = std::make_shared<det_session>();
     w->m = m;
     w->ctx = ctx;
     w->max_tokens = std::max(ac.cap, sc->dec ? sc->dec->score_stride : 0);
@@ -3137,6 +3116,7 @@ bool layer_decode_fused(det_scratch* sc, uint64_t l, const int32_t* input, const
     fused_alloc(w.get(), w->max_tokens);
     sc->dec = std::move(w);
   }
+  if (ctx->capturing) ctx->recorded.push_back(sc->dec);
   det_session* ws = scratch_rows(sc, 1);
   det_session* d = sc->dec.get();
   const auto& F = m->fused[l];
@@ -3265,12 +3245,6 @@ int det_ctx_create(int device, det_ctx_t** out) {
 void det_ctx_destroy(det_ctx_t* ctx) {
   if (!ctx) return;
   (void)hipStreamSynchronize(ctx->stream);
-  if (ctx->limbs) (void)hipFree(ctx->limbs);
-  if (ctx->gemm_a) (void)hipFree(ctx->gemm_a);
-  if (ctx->gemm_planes) (void)hipFree(ctx->gemm_planes);
-  if (ctx->attn_work) (void)hipFree(ctx->attn_work);
-  if (ctx->rows_work) (void)hipFree(ctx->rows_work);
-  if (ctx->argmax_scratch) (void)hipFree(ctx->argmax_scratch);
   if (ctx->argmax_out) (void)hipFree(ctx->argmax_out);
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
@@ -3331,6 +3305,9 @@ int det_ctx_capture_end(det_ctx_t* ctx, det_graph_t** out) {
     if (!ctx->capturing) bail("det_ctx_capture_end: no capture in progress (a failed call ends it)");
     ctx->capturing = false;
     auto g = std::make_unique<det_graph>();
+    g->scratch.swap(ctx->recorded);
+    for (const DevRef& r : {ctx->limbs.mem, ctx->gemm_a.mem, ctx->gemm_planes.mem, ctx->attn_work.mem})
+      if (r) g->scratch.push_back(r);
     HIPC(hipStreamEndCapture(ctx->stream, &g->graph));
     HIPC(hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0));
     *out = g.release();
@@ -3382,10 +3359,10 @@ void det_matrix_free(det_matrix_t* m) {
 }
 
 int det_linear(det_ctx_t* ctx, const det_matrix_t* w, const int32_t* act, int32_t* out) {
-  return guarded(ctx, [&] { det::launch_linear(w->m, act, 1, w->m.cols, out, w->m.rows, nullptr, ctx->limbs, ctx->stream); });
+  return guarded(ctx, [&] { det::launch_linear(w->m, act, 1, w->m.cols, out, w->m.rows, nullptr, ctx->limbs.get(), ctx->stream); });
 }
 int det_linear_acc_i64(det_ctx_t* ctx, const det_matrix_t* w, const int32_t* act, int64_t* acc) {
-  return guarded(ctx, [&] { det::launch_linear(w->m, act, 1, w->m.cols, nullptr, w->m.rows, acc, ctx->limbs, ctx->stream); });
+  return guarded(ctx, [&] { det::launch_linear(w->m, act, 1, w->m.cols, nullptr, w->m.rows, acc, ctx->limbs.get(), ctx->stream); });
 }
 int det_linear_slab(det_ctx_t* ctx, const det_matrix_t* w, uint64_t m, const int32_t* act, int32_t* out) {
   return guarded(ctx, [&] { ctx->linear(w->m, act, m, w->m.cols, out, w->m.rows, nullptr); });

@@ -292,3 +292,48 @@ def test_layer_decode_routes_agree(ctx, prompt, window, donor):
     assert len(a[0]) == len(b[0]) and all(np.array_equal(p, q) for p, q in zip(a[0], b[0]))
     for (k0, v0), (k1, v1) in zip(a[1], b[1]):
         assert np.array_equal(k0, k1) and np.array_equal(v0, v1)
+
+
+def test_recorded_layer_calls_keep_their_scratch():
+    """A graph of layer calls replays correctly after later calls on the same scratch and context have replaced
+    every scratch buffer it uses with a larger one: the decode buffers (a larger cache), the row buffers and the
+    GEMM, GEMV and attention areas (more rows, a wider matrix)."""
+    cfg = synthetic.e4b_config(layers=2, vocab=512, sliding_window=64)
+    cfg["text_config"].update({"hidden_size": 128, "intermediate_size": 256, "head_dim": 64,
+                               "num_attention_heads": 4, "num_key_value_heads": 1})
+    own = rd.Context(0)  # (scratch of its own, so that it starts small)
+    model = rd.Model(own, cfg)
+    for name, v, s in fixtures.custom_model(cfg, seed=9):
+        model.set_tensor(name, v, s)
+    model.finalize()
+    assert model.fused_decode
+    rng = np.random.default_rng(4)
+    acts = lambda *shape: np.rint(rng.normal(size=shape) * 65536).astype(np.int32)  # noqa: E731
+    ops, n = rd.LayerOps(model), 20
+    prompt, row = own.to_device(acts(n, 128)), own.to_device(acts(128))
+    mid, out, wide = own.empty((n, 128)), own.empty(128), own.empty(1000)
+    cache = rd.KvCache(model, 0, 64)
+    q, s = synthetic.fast_int8_matrix(3, 1000, 128, 16)
+    mat = own.upload_matrix(q, s)
+
+    def calls():
+        ops.layer_prefill(0, prompt, n, None, None, cache, mid)  # GEMM, attention and row scratch
+        ops.layer_decode(0, row, None, cache, None, n, out)      # decode scratch
+        own.det_linear_into(mat, out, wide)                      # GEMV scratch
+
+    calls()  # (their scratch exists now)
+    want = [b.numpy().copy() for b in (mid, out, wide)]
+    graph = own.capture(calls)
+    big, rows = rd.KvCache(model, 1, 3000), 700
+    many, more = own.to_device(acts(rows, 128)), own.empty((rows, 128))
+    wq, ws = synthetic.fast_int8_matrix(4, 32, 40000, 16)
+    filler = []
+    for i in range(3):
+        ops.layer_prefill(1, many, rows, None, None, big, more)
+        ops.layer_decode(1, row, None, big, None, rows, more)
+        own.upload_matrix(wq, ws)
+        filler.append(own.to_device(acts(1 << 20)))  # takes freed memory, if any was freed
+        for b in (mid, out, wide):
+            b.upload(np.zeros(b.shape, np.int32))
+        graph.launch()
+        assert all(np.array_equal(w, b.numpy()) for w, b in zip(want, (mid, out, wide))), i
