@@ -112,16 +112,34 @@ struct det_ctx {
   }
   // The MFMA attention's work area for a (null where that form does not
   // apply or would need more than kAttnWorkMax bytes even in query chunks: the
-  // vector-ALU kernel runs then, and also for a call whose unchunked form
-  // passes the bound when a recording stream keeps the area from growing).
+  // vector-ALU kernel runs then, and also where a call whose unchunked form
+  // passes the bound finds the area too small and cannot make it larger). The
+  // area is as large as unchunked calls of these rows take, up to the bound:
+  // what a chunked or windowed call needs does not grow with its rows (3584
+  // rows of 8/2 heads of 256 need more than 3712 do), and an area of that size
+  // would not cover a shorter call that is recorded after a longer one. (A
+  // 64th on top covers the per-row words of any other head shape whose score
+  // rows and limbs fit.)
   static constexpr uint64_t kAttnWorkMax = uint64_t(512) << 20;
   void attach_attn_work(det::AttnArgs& a) {
-    const uint64_t bytes = det::attn_mfma_bytes(a);
+    const uint64_t need = det::attn_mfma_bytes(a);
     a.work = nullptr;
     a.work_bytes = 0;
-    if (bytes == 0 || bytes > kAttnWorkMax) return;
-    if (bytes > attn_work.bytes && capturing && det::attn_mfma_unchunked_bytes(a) > kAttnWorkMax) return;
-    grow(attn_work, bytes, "attention");
+    if (need == 0 || need > kAttnWorkMax) return;
+    const uint64_t whole = det::attn_mfma_unchunked_bytes(a);
+    const uint64_t size = std::min(whole + whole / 64, kAttnWorkMax);
+    if (size > attn_work.bytes && !capturing) {
+      try {
+        grow(attn_work, size, "attention");
+      } catch (const Status&) {
+        if (whole <= kAttnWorkMax) throw;
+        (void)hipGetLastError();
+      }
+    }
+    if (need > attn_work.bytes) {
+      if (whole > kAttnWorkMax) return;
+      grow_check("attention");
+    }
     a.work = attn_work.get();
     a.work_bytes = attn_work.bytes;
   }

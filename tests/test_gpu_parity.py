@@ -261,6 +261,28 @@ def test_attention_causal_tiles(ctx, nq, nrows, nh, nkv, hd, window, wide):
             assert np.array_equal(got[t, h * hd:(h + 1) * hd], o), (t, h)
 
 
+@pytest.mark.parametrize("warm,warm_window,n", [(3712, 0, 3584), (700, 48, 700), (5000, 0, 4500)])
+def test_attention_recorded_after_a_longer_call(warm, warm_window, n):
+    """A call of at least as many rows, windowed or not, leaves scratch that a recorded call of fewer rows fits:
+    one of nearly three thousand to 3712 rows (whose chunks round up), one without the window, and one past the
+    work area's bound, which may always be recorded."""
+    ctx, heads, kv, hd = rd.Context(0), 8, 2, 256
+    rng = np.random.default_rng(n)
+    q, k, v = (ctx.to_device(np.rint(rng.normal(size=(warm, h * hd)) * 65536).astype(np.int32)) for h in (heads, kv, kv))
+    out = ctx.empty((warm, heads * hd))
+    ctx.attention(q, k, v, warm, warm, heads, kv, hd, warm_window, out)
+    graph = ctx.capture(lambda: ctx.attention(q, k, v, n, n, heads, kv, hd, 0, out))
+    want = None
+    for i in range(3):
+        out.upload(np.zeros(out.shape, np.int32))
+        graph.launch()
+        got = out.numpy()[:n].copy()
+        if want is None:
+            ctx.attention(q, k, v, n, n, heads, kv, hd, 0, out)
+            want = out.numpy()[:n].copy()
+        assert np.array_equal(got, want), i
+
+
 @pytest.mark.parametrize("n", [1, 5, 1023, 1024, 1025, 262144])
 def test_argmax_first(ctx, n):
     rng = np.random.default_rng(n)
