@@ -1057,26 +1057,39 @@ struct det_session {
     if (graph) (void)hipGraphDestroy(graph);
     for (void* p : owned) (void)hipFree(p);
   }
-  // Buffers are cut from device allocations of at least slab_bytes: a session
-  // is about forty buffers, and an allocation and a free of each cost more
-  // than the first decode steps.
-  uint64_t slab_bytes = uint64_t(1) << 20, slab_left = 0;
+  // A session is about forty buffers, and an allocation and a free of each
+  // cost more than the first decode steps: build() runs the code that
+  // allocates them twice, first to add up their sizes and then to cut them
+  // from one device allocation of exactly that size.
+  bool sizing = false;
+  uint64_t slab_bytes = 0;
   uint8_t* slab = nullptr;
   template <class T>
   T* alloc(uint64_t n) {
-    const uint64_t bytes = (std::max<uint64_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
-    if (bytes > slab_left) {
-      const uint64_t size = std::max(bytes, slab_bytes);
-      void* p = nullptr;
-      HIPC(hipMalloc(&p, size));
-      owned.push_back(p);
-      slab = static_cast<uint8_t*>(p);
-      slab_left = size;
+    uint64_t bytes = 0, total = 0;
+    if (__builtin_mul_overflow(std::max<uint64_t>(n, 1), uint64_t(sizeof(T)), &bytes) ||
+        __builtin_add_overflow(slab_bytes, bytes, &total) || total > UINT64_MAX - 255)
+      throw Status(3, "session buffers: out of memory");
+    bytes = round_up(bytes, 256);
+    if (sizing) {
+      slab_bytes = round_up(total, 256);
+      return nullptr;
     }
     T* r = reinterpret_cast<T*>(slab);
     slab += bytes;
-    slab_left -= bytes;
     return r;
+  }
+  template <class F>
+  void build(F&& cuts) {
+    sizing = true;
+    cuts();
+    sizing = false;
+    void* p = nullptr;
+    HIPC(hipMalloc(&p, slab_bytes));
+    owned.push_back(p);
+    slab = static_cast<uint8_t*>(p);
+    slab_bytes = 0;
+    cuts();
   }
 };
 
@@ -1106,7 +1119,8 @@ struct det_scratch {
 
 namespace {
 
-// The fused decode step's buffers, for attention windows of up to T rows.
+// The fused decode step's buffers, for attention windows of up to T rows (in
+// det_session::build).
 void fused_alloc(det_session* s, uint64_t T) {
   det_model* m = s->m;
   const uint64_t H = m->hidden;
@@ -1128,12 +1142,14 @@ void fused_alloc(det_session* s, uint64_t T) {
   s->kpad_x = m->fused[0].qkv.kpad;
   s->limbs_x = s->alloc<int8_t>(4 * s->kpad_x);
   s->limbs_ff = s->alloc<int8_t>(4 * kff);
-  hipStream_t zst = m->ctx->stream;  // stream-ordered before any step (not inside a graph)
-  HIPC(hipMemsetAsync(s->limbs_x, 0, 4 * s->kpad_x, zst));
-  HIPC(hipMemsetAsync(s->limbs_ff, 0, 4 * kff, zst));
-  HIPC(hipMemsetAsync(s->qkv_acc, 0, fr * 8, zst));
-  HIPC(hipMemsetAsync(s->o_acc, 0, H * 8, zst));
-  HIPC(hipMemsetAsync(s->ff_acc, 0, H * 8, zst));
+  auto clear = [&](void* p, uint64_t bytes) {  // stream-ordered before any step (not inside a graph)
+    if (!s->sizing) HIPC(hipMemsetAsync(p, 0, bytes, m->ctx->stream));
+  };
+  clear(s->limbs_x, 4 * s->kpad_x);
+  clear(s->limbs_ff, 4 * kff);
+  clear(s->qkv_acc, fr * 8);
+  clear(s->o_acc, H * 8);
+  clear(s->ff_acc, H * 8);
   s->scores = s->alloc<int32_t>(nh * T);
   s->attn_keys = s->alloc<int64_t>(nh * ((T + det::kAttnScoreRows - 1) / det::kAttnScoreRows));
   s->attn_stats = s->alloc<det::AttnStat>(nh);
@@ -1149,7 +1165,7 @@ void fused_alloc(det_session* s, uint64_t T) {
     s->ple_pp = s->alloc<int32_t>(rows);
     s->ple_g = s->alloc<int32_t>(m->ple_dim);
     s->ple_acc = s->alloc<int64_t>(H);
-    HIPC(hipMemsetAsync(s->ple_acc, 0, H * 8, zst));
+    clear(s->ple_acc, H * 8);
   }
 }
 
@@ -1235,21 +1251,10 @@ struct PrefillRows {
   }
 };
 
-// Allocates a session's buffers: its activation rows (max_tokens of them, or
-// one with `one_row`); with_state adds the per-layer KV caches and the fused
-// decode step's buffers (a workspace for the layer-level entry points has
-// neither).
-void session_alloc(det_session* s, bool with_state = true, bool one_row = false) {
+// The buffers of session_alloc.
+void session_buffers(det_session* s, bool with_state, bool one_row) {
   det_model* m = s->m;
-  s->ctx = m->ctx;
   const uint64_t T = s->max_tokens, H = m->hidden;
-  auto cache_rows = [&](const GLayer& L) {
-    if (!L.cache_sliding_window) return T;
-    return std::max<uint64_t>(std::min<uint64_t>(*L.cache_sliding_window, T), 1);
-  };
-  if (with_state)
-    for (const GLayer& L : m->layers)
-      if (!L.donor) s->slab_bytes += 2 * cache_rows(L) * L.num_kv_heads * L.head_dim * 4 + 512;
   row_buffers(s, one_row ? 1 : T, [&](uint64_t b) -> void* { return s->alloc<int8_t>(b); });
   s->logits = s->alloc<int32_t>(m->vocab);
   s->dec_in = s->alloc<int32_t>(H);
@@ -1265,10 +1270,19 @@ void session_alloc(det_session* s, bool with_state = true, bool one_row = false)
     c.row_w = L.num_kv_heads * L.head_dim;
     if (L.donor) continue;  // shared layers never hold det data
     c.ring = L.cache_sliding_window.has_value();
-    c.cap = cache_rows(L);
+    c.cap = c.ring ? std::max<uint64_t>(std::min<uint64_t>(*L.cache_sliding_window, T), 1) : T;
     c.k = s->alloc<int32_t>(c.cap * c.row_w);
     c.v = s->alloc<int32_t>(c.cap * c.row_w);
   }
+}
+
+// Allocates a session's buffers: its activation rows (max_tokens of them, or
+// one with `one_row`); with_state adds the per-layer KV caches and the fused
+// decode step's buffers (a workspace for the layer-level entry points has
+// neither).
+void session_alloc(det_session* s, bool with_state = true, bool one_row = false) {
+  s->ctx = s->m->ctx;
+  s->build([&] { session_buffers(s, with_state, one_row); });
 }
 
 // The logical rows of a cache (oldest to newest) copied to the host as
@@ -3131,7 +3145,7 @@ bool layer_decode_fused(det_scratch* sc, uint64_t l, const int32_t* input, const
     w->ctx = ctx;
     w->max_tokens = std::max(ac.cap, sc->dec ? sc->dec->score_stride : 0);
     w->kv.assign(m->layers.size(), GKv());
-    fused_alloc(w.get(), w->max_tokens);
+    w->build([&] { fused_alloc(w.get(), w->max_tokens); });
     sc->dec = std::move(w);
   }
   if (ctx->capturing) ctx->recorded.push_back(sc->dec);

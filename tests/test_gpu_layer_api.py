@@ -337,3 +337,30 @@ def test_recorded_layer_calls_keep_their_scratch():
             b.upload(np.zeros(b.shape, np.int32))
         graph.launch()
         assert all(np.array_equal(w, b.numpy()) for w, b in zip(want, (mid, out, wide))), i
+
+
+def free_memory() -> int:
+    """Free bytes of the device, from the HIP runtime that the library is linked against."""
+    free, total = rd.C.c_size_t(), rd.C.c_size_t()
+    assert rd.lib().hipMemGetInfo(rd.C.byref(free), rd.C.byref(total)) == 0
+    return free.value
+
+
+def test_session_memory_is_its_buffers():
+    """A session takes its caches and step buffers and no more, also where the vocabulary row alone is a MiB."""
+    cfg = synthetic.e4b_config(layers=2, vocab=262144, sliding_window=64)
+    cfg["text_config"].update({"hidden_size": 128, "intermediate_size": 256, "head_dim": 64, "num_attention_heads": 4,
+                               "num_key_value_heads": 2, "layer_types": ["full_attention"] * 2})
+    own = rd.Context(0)
+    model = rd.Model(own, cfg)
+    for name, v, s in fixtures.custom_model(cfg, seed=2):
+        model.set_tensor(name, v, s)
+    model.finalize()
+    tokens = 200_000
+    kv = 2 * 2 * tokens * 2 * 64 * 4  # layers, keys and values, rows, KV heads x head dim, int32
+    rest = 4 * tokens * 4 + 262144 * 4  # score rows, logits
+    before = free_memory()
+    session = model.session(tokens)
+    used = before - free_memory()
+    assert kv <= used <= kv + rest + (8 << 20), (used, kv)
+    del session
