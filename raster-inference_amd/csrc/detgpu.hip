@@ -1282,6 +1282,8 @@ void session_buffers(det_session* s, bool with_state, bool one_row) {
 // neither).
 void session_alloc(det_session* s, bool with_state = true, bool one_row = false) {
   s->ctx = s->m->ctx;
+  // (past this no row or cache fits any device, and sizes would wrap around)
+  if (s->max_tokens > uint64_t(1) << 36) throw Status(3, "session buffers: out of memory");
   s->build([&] { session_buffers(s, with_state, one_row); });
 }
 

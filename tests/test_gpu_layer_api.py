@@ -364,3 +364,22 @@ def test_session_memory_is_its_buffers():
     used = before - free_memory()
     assert kv <= used <= kv + rest + (8 << 20), (used, kv)
     del session
+
+
+@pytest.mark.parametrize("tokens", [2**37, 2**54, 2**60, 2**62, 2**64 - 1])
+@pytest.mark.parametrize("sliding", [False, True])
+def test_session_too_large_for_any_device_is_refused(ctx, tokens, sliding):
+    """Sizes that wrap around 64 bits (2^54 rows of 256 words, 2^60 score rows of 4 heads) are refused like any
+    other session that does not fit, with and without caches that grow with it."""
+    cfg = synthetic.e4b_config(layers=2, vocab=512, sliding_window=16)
+    cfg["text_config"].update({"hidden_size": 128, "intermediate_size": 256, "head_dim": 64, "num_attention_heads": 4,
+                               "num_key_value_heads": 4})
+    if sliding:
+        cfg["text_config"]["layer_types"] = ["sliding_attention"] * 2
+    model = rd.Model(ctx, cfg)
+    for name, v, s in fixtures.custom_model(cfg, seed=2):
+        model.set_tensor(name, v, s)
+    model.finalize()
+    with pytest.raises(rd.DetError, match="out of memory"):
+        model.session(tokens)
+    model.session(64).prefill([1, 2, 3])
