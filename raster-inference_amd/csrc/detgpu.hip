@@ -1593,7 +1593,7 @@ bool layer_prefill(det_session* ws, const GLayer& L, uint64_t n, GKv* own, const
   hipStream_t st = ctx->stream;
   const uint64_t H = m->hidden;
   if (n == 0) bail("transformer layer execution requires at least one activation row");
-  if (n > ws->max_tokens) bail("activation rows exceed the scratch capacity");
+  if (n > ws->row_cap) bail("activation rows exceed the scratch capacity");
   if (!donor && !own) bail("transformer prefill layer needs its own cache or a donor cache");
   if (!normed_ready) det::launch_rmsnorm_to(ws->normed, ws->x, n, H, H, L.in_ln, L.eps, st);
   const uint64_t kw = L.num_kv_heads * L.head_dim;
