@@ -56,7 +56,7 @@ struct AttnDecArgs {
   int32_t* v;
   const StepState* st;
   uint64_t cap, window;
-  uint64_t max_rows;  // row stride of the scores scratch (>= cap)
+  uint64_t max_rows;  // row stride of the scores scratch (>= every window)
   int ring;
   uint32_t hd, nh, nkv;
   int32_t* scores;  // scratch [nh][max_rows]

@@ -1112,7 +1112,7 @@ struct det_scratch {
   det_model* m = nullptr;
   det_ctx* ctx = nullptr;  // m->ctx, kept so that freeing the scratch does not read the model
   std::shared_ptr<det_session> ws;
-  // the fused step's buffers for det_layer_decode, for caches of up to
+  // the fused step's buffers for det_layer_decode, for windows of up to
   // dec->score_stride rows
   std::shared_ptr<det_session> dec;
 };
@@ -3139,13 +3139,14 @@ bool layer_decode_fused(det_scratch* sc, uint64_t l, const int32_t* input, const
     return false;
   const uint64_t rows = ac.ring ? std::min(position + 1, ac.cap) : position + 1;
   if ((L.sliding ? std::min<uint64_t>(rows, *L.sliding_window) : rows) > det::kMaxAttentionRows) return false;
-  if (!sc->dec || sc->dec->score_stride < ac.cap) {
+  const uint64_t span = std::min(ac.cap, det::kMaxAttentionRows);  // (no window passes either)
+  if (!sc->dec || sc->dec->score_stride < span) {
     if (ctx->capturing) return false;  // (no allocation while the stream records)
     HIPC(hipStreamSynchronize(st));
     auto w = std::make_shared<det_session>();
     w->m = m;
     w->ctx = ctx;
-    w->max_tokens = std::max(ac.cap, sc->dec ? sc->dec->score_stride : 0);
+    w->max_tokens = std::max(span, sc->dec ? sc->dec->score_stride : 0);
     w->kv.assign(m->layers.size(), GKv());
     w->build([&] { fused_alloc(w.get(), w->max_tokens); });
     sc->dec = std::move(w);
@@ -3162,10 +3163,13 @@ bool layer_decode_fused(det_scratch* sc, uint64_t l, const int32_t* input, const
   a.k = ac.k;
   a.v = ac.v;
   a.own_cache = !donor;
-  a.cap = ac.cap;
+  // A linear cache is as long as its rows so far: the kernels' grids cover a.cap
+  // rows, and one block per 32 or 128 rows of a million-row cache took 132 us
+  // at 16 rows (51 this way).
+  a.cap = ac.ring ? ac.cap : rows;
   a.ring = ac.ring;
-  a.scores_in_lds = (L.num_heads / L.num_kv_heads) * ac.cap * 4 <= 32768;
-  a.lds_stride = ac.cap;
+  a.scores_in_lds = (L.num_heads / L.num_kv_heads) * a.cap * 4 <= 32768;
+  a.lds_stride = a.cap;
   det::launch_dec_attention(a, st);
   det::launch_gemv_decode_acc(*L.o, d->attn_acc, true, d->o_acc, st);
   det::DecNormIn ni;

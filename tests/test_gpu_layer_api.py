@@ -383,3 +383,28 @@ def test_session_too_large_for_any_device_is_refused(ctx, tokens, sliding):
     with pytest.raises(rd.DetError, match="out of memory"):
         model.session(tokens)
     model.session(64).prefill([1, 2, 3])
+
+
+def test_layer_decode_scratch_is_bounded_by_the_window():
+    """A decode in a cache of millions of rows takes scratch for the longest window there is, not for the cache, and
+    gives what a small cache gives."""
+    cfg = synthetic.e4b_config(layers=2, vocab=512, sliding_window=64)
+    cfg["text_config"].update({"hidden_size": 128, "intermediate_size": 256, "head_dim": 64, "num_attention_heads": 4,
+                               "num_key_value_heads": 1})
+    own = rd.Context(0)
+    model = rd.Model(own, cfg)
+    for name, v, s in fixtures.custom_model(cfg, seed=3):
+        model.set_tensor(name, v, s)
+    model.finalize()
+    rng = np.random.default_rng(6)
+    rows, row = (own.to_device(np.rint(rng.normal(size=(n, 128)) * 65536).astype(np.int32)) for n in (30, 1))
+    got = []
+    for cap in (64, 4_000_000):
+        ops, cache, out = rd.LayerOps(model), rd.KvCache(model, 1, cap), own.empty((30, 128))
+        ops.layer_prefill(1, rows, 30, None, None, cache, out)
+        before = free_memory()
+        for pos in range(30, 34):
+            ops.layer_decode(1, row, None, cache, None, pos, out)
+            got.append(out.numpy()[0].copy())
+        assert before - free_memory() <= 8 << 20, cap
+    assert all(np.array_equal(a, b) for a, b in zip(got[:4], got[4:]))
