@@ -316,7 +316,7 @@ struct AttnMfmaArgs {
   int64_t* qsum;
   int64_t* ksum;
   int64_t* vblk;
-  uint32_t* vwide;  // per KV head and key substep: the V limbs take the four-limb split
+  uint32_t* vwide;  // per KV head, 256 head dims and key substep: the V limbs take the four-limb split
   const int32_t* v;
   uint64_t kv_ld;
   // the chunk of queries [t0, t0 + crow_used) whose scores (crow rows per

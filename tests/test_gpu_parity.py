@@ -223,28 +223,10 @@ def test_attention_causal(ctx, nq, nh, nkv, hd, window, mag):
     assert np.array_equal(out.numpy(), oracle_attention(q, k, v, nq, nq, nh, nkv, hd, window))
 
 
-@pytest.mark.parametrize("nq,nrows,nh,nkv,hd,window,wide", [
-    (16, 16, 4, 1, 64, 0, False),       # one tile of queries and keys
-    (31, 47, 3, 1, 64, 0, False),       # three heads per KV head, rows past the queries
-    (515, 515, 8, 2, 256, 100, False),  # one key past a score span; windows that start inside a substep
-    (2300, 2300, 8, 2, 256, 0, True),   # two chunks of queries, more than 2048 keys, two key tiles per wave
-    (1100, 1100, 8, 4, 128, 1030, True),
-])
-def test_attention_causal_tiles(ctx, nq, nrows, nh, nkv, hd, window, wide):
-    """Normalised rows (three limbs) with single rows, keys and values past 24 bits (`wide`, int32
-    extremes among them), a query whose softmax is one key of weight 65536, and equal maxima."""
-    rng = np.random.default_rng(nq + hd)
-    q, k, v = (np.rint(rng.normal(size=(n, h * hd)) * 65536).astype(np.int32)
-               for n, h in ((nq, nh), (nrows, nkv), (nrows, nkv)))
-    k[3], v[5, :hd] = k[2], -65536
-    q[9] = np.tile(k[4, :hd], nh) * 3  # its own key far above the rest
-    if wide:
-        k[70, 5], k[900, 7], v[130, 3], v[700, 1], q[300, 2] = 1 << 23, -(1 << 31), (1 << 31) - 1, -(1 << 24), 1 << 25
-    out = ctx.empty((nq, nh * hd))
-    ctx.attention(ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), nq, nrows, nh, nkv, hd, window, out)
-    got, L, g = out.numpy(), oracle_lib.lib(), nh // nkv
-    picks = {0, 9, 15, nq - 1, nq // 2, 70, 71, 300, 901, 1023, 1050, 2047, 2048}
-    for t in sorted(x for x in picks if x < nq):
+def check_attention_rows(got, q, k, v, picks, nh, nkv, hd, window):
+    """Rows `picks` of causal attention against the oracle."""
+    L, g = oracle_lib.lib(), nh // nkv
+    for t in sorted(picks):
         start = max(0, t + 1 - window) if window else 0
         for h in range(nh):
             cols = slice(h // g * hd, (h // g + 1) * hd)
@@ -259,6 +241,60 @@ def test_attention_causal_tiles(ctx, nq, nrows, nh, nkv, hd, window, wide):
             L.orc_attention_softmax(oracle_lib.ptr(logits), len(ks), oracle_lib.ptr(w))
             L.orc_attention_weighted_sum(oracle_lib.ptr(w), oracle_lib.ptr(vs), len(ks), hd, oracle_lib.ptr(o))
             assert np.array_equal(got[t, h * hd:(h + 1) * hd], o), (t, h)
+
+
+def attention_rows(seed, nq, nrows, nh, nkv, hd):
+    """Normalised q, k, v rows: equal maxima, and a query whose softmax is one key of weight 65536."""
+    rng = np.random.default_rng(seed)
+    q, k, v = (np.rint(rng.normal(size=(n, h * hd)) * 65536).astype(np.int32)
+               for n, h in ((nq, nh), (nrows, nkv), (nrows, nkv)))
+    k[3], v[5, :hd] = k[2], -65536
+    q[9] = np.tile(k[4, :hd], nh) * 3  # its own key far above the rest
+    return q, k, v
+
+
+@pytest.mark.parametrize("nq,nrows,nh,nkv,hd,window,wide", [
+    (16, 16, 4, 1, 64, 0, False),       # one tile of queries and keys
+    (31, 47, 3, 1, 64, 0, False),       # three heads per KV head, rows past the queries
+    (515, 515, 8, 2, 256, 100, False),  # one key past a score span; windows that start inside a substep
+    (2300, 2300, 8, 2, 256, 0, True),   # more than 2048 keys in one row
+    (1100, 1100, 8, 4, 128, 1030, True),
+    (1026, 1026, 4, 2, 64, 1024, False),  # windows as long as the one-wave softmax takes
+    (1027, 1027, 4, 2, 64, 1025, False),  # and one key longer
+    (1025, 1025, 3, 1, 192, 0, True),     # six waves of scores; one row past 1024 keys
+    (950, 990, 2, 2, 320, 200, True),     # two 256-dim parts of V, the second with one dim group
+])
+def test_attention_causal_tiles(ctx, nq, nrows, nh, nkv, hd, window, wide):
+    """Normalised rows (three limbs) with single rows, keys and values past 24 bits (`wide`, int32
+    extremes among them), a query whose softmax is one key of weight 65536, and equal maxima."""
+    q, k, v = attention_rows(nq + hd, nq, nrows, nh, nkv, hd)
+    if wide:
+        k[70, 5], k[900, 7], v[130, 3], v[700, 1], q[300, 2] = 1 << 23, -(1 << 31), (1 << 31) - 1, -(1 << 24), 1 << 25
+        v[400, nkv * hd - 1] = 1 << 24
+    out = ctx.empty((nq, nh * hd))
+    ctx.attention(ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), nq, nrows, nh, nkv, hd, window, out)
+    picks = {0, 9, 15, nq - 1, nq // 2, 70, 71, 300, 901, 1023, 1050, 2047, 2048}
+    check_attention_rows(out.numpy(), q, k, v, {x for x in picks if x < nq}, nh, nkv, hd, window)
+
+
+@pytest.mark.parametrize("n,nh,nkv,hd,window,edges,wide", [
+    (3105, 8, 2, 256, 0, [2656], False),               # 2656 queries, then 449
+    (5300, 8, 2, 64, 1500, [5216], False),             # windows that reach back over the boundary
+    (6500, 4, 1, 64, 0, [2560, 5120], True),           # values of four limbs past the first 64 substeps
+    (10500, 1, 1, 64, 0, [6336], True),                # rows longer than four waves' softmax takes
+])
+def test_attention_causal_chunks_of_queries(ctx, n, nh, nkv, hd, window, edges, wide):
+    """Score rows past 256 MB go in chunks of queries: rows on both sides of each boundary and in the last tile."""
+    per = nh * 4 * (min(-(-n // 64) * 64, (window + 94) // 64 * 64 + 64) if window else -(-n // 64) * 64)
+    rows = max((256 << 20) // per, 32) // 32 * 32
+    assert edges == list(range(rows, n, rows))  # (where the chunks of this case begin)
+    q, k, v = attention_rows(n, n, n, nh, nkv, hd)
+    if wide:
+        v[4500, 3], v[4800, 1], v[n - 20, 5], k[5200, 7], q[n - 3, 2] = 1 << 24, -(1 << 31), (1 << 31) - 1, 1 << 23, 1 << 25
+    out = ctx.empty((n, nh * hd))
+    ctx.attention(ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), n, n, nh, nkv, hd, window, out)
+    picks = {9, 4801, n - 20, n - 3, n - 1} | {e + d for e in edges for d in (-1, 0, 1, 33)}
+    check_attention_rows(out.numpy(), q, k, v, {x for x in picks if x < n}, nh, nkv, hd, window)
 
 
 @pytest.mark.parametrize("warm,warm_window,n", [(3712, 0, 3584), (700, 48, 700), (5000, 0, 4500)])
