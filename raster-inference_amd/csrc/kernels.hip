@@ -3172,18 +3172,23 @@ static bool gemm_small(const DevMatrix& W, uint64_t m) {
 // row counts below the first shape's (20480-row gate/up with its limb
 // expansion, against 128 x 128 blocks): 32 tokens x 80 rows at 17 to 32 rows,
 // 20.4 -> 17.9 us; 32 tokens x 160 rows at 33 to 64, 24.8 -> 22.4 us (64 x 80
-// on four waves 29.6 us: each reads eight operands for fifteen MFMAs).
+// on four waves 29.6 us: each reads eight operands for fifteen MFMAs). The
+// first from two K steps on (one step: 8.7 -> 8.8 us). The second only where
+// the blocks divide over the eight XCDs, since only then do the two token
+// blocks of a weight tile meet in one L2: 19456 x 4096 at 64 rows, 244 blocks,
+// 30.2 us in 128 x 128 blocks and 32.0 in these; 18432 x 4096, 232 blocks,
+// 30.3 and 27.4. They serve matrices of about 18.4 to 20.5 thousand rows.
 // At 512 and 2048 rows the grids take several rounds and none applies.
 enum class PadShape { kNone, k64x160, k32x48, k16x80, k32x80, k32x160 };
 static PadShape gemm_pad_shape(const DevMatrix& W, uint64_t m) {
   if (W.storage != kInt8 || W.planes != 1 || W.kpad > 32 * 128) return PadShape::kNone;
   const uint64_t tiles = (W.rows + 15) / 16, cus = device_cus();
+  auto blocks = [&](uint64_t tokens, uint64_t tb) { return ((m + tokens - 1) / tokens) * ((tiles + tb - 1) / tb); };
   auto fills = [&](uint64_t tokens, uint64_t tb) {
-    const uint64_t blocks = ((m + tokens - 1) / tokens) * ((tiles + tb - 1) / tb);
-    return blocks <= cus && blocks * 10 >= cus * 9;
+    return blocks(tokens, tb) <= cus && blocks(tokens, tb) * 10 >= cus * 9;
   };
-  if (m > 16 && m <= 32 && fills(32, 5)) return PadShape::k32x80;
-  if (m > 32 && m <= 64 && fills(32, 10)) return PadShape::k32x160;
+  if (m > 16 && m <= 32 && W.kpad >= 256 && fills(32, 5)) return PadShape::k32x80;
+  if (m > 32 && m <= 64 && blocks(32, 10) % 8 == 0 && fills(32, 10)) return PadShape::k32x160;
   if (fills(64, 10)) return PadShape::k64x160;
   if (fills(32, 3)) return PadShape::k32x48;
   if (fills(16, 5)) return PadShape::k16x80;

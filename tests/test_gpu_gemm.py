@@ -146,12 +146,14 @@ def test_gemm_unaligned_activation_rows(ctx):
 # not divide over the waves: (128 | 100 | 65, 20480, 2560) 64 x 160 blocks
 # (the stacked gate/up slab; 65 rows: one token in the last block),
 # (128 | 100 | 97, 3072, 2560) 32 x 48 blocks (q/k/v), (128 | 113, 2560, 2048)
-# 16 x 80 blocks (o; 113 rows: one token in the last group).
+# 16 x 80 blocks (o; 113 rows: one token in the last group), (17 | 32, 20480)
+# 32 x 80 and (33 | 64, 20480) 32 x 160 blocks; neither for one K step (20,
+# 20480, 100) and for blocks that do not divide over the XCDs (40, 19456, 300).
 @pytest.mark.parametrize("m,n,k", [(128, 3072, 2560), (100, 3072, 2560), (97, 3072, 2560), (64, 2560, 10240),
                                    (48, 2560, 2048), (128, 2560, 2048), (113, 2560, 2048), (256, 16384, 512),
                                    (300, 13100, 2600), (128, 20480, 2560), (100, 20480, 2560), (65, 20480, 2560),
                                    (160, 16384, 2560), (17, 20480, 2560), (32, 20475, 2560), (33, 20480, 2500),
-                                   (64, 20480, 4096)])
+                                   (64, 20480, 4096), (20, 20480, 100), (40, 19456, 300)])
 def test_gemm_e4b_shapes_match_gemv_rows(ctx, m, n, k):
     q, s = synthetic.fast_int8_matrix(n * 31 + k, n, k, 256)
     acts = act_slab(m, k, seed=n + k)
