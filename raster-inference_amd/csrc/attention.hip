@@ -682,7 +682,9 @@ __device__ __forceinline__ void wsum_loop(const WsumSrc<WsumShape<GB, VL>::RPW>&
       }
   }
 }
-template <int GB>
+// OVER: the outputs share memory with V, whose argmax rows then come from its
+// limbs (as a branch of one kernel this cost layers of 16 to 800 rows 2-3 %).
+template <int GB, bool OVER>
 __global__ __launch_bounds__(512) void k_attn_wsum_mfma(AttnMfmaArgs a) {
   constexpr int NA = GB, RPW = WsumShape<GB, 3>::RPW;
   extern __shared__ __attribute__((aligned(16))) int8_t ring[];  // [stage][weight halves, V limbs][lane]
@@ -740,7 +742,16 @@ __global__ __launch_bounds__(512) void k_attn_wsum_mfma(AttnMfmaArgs a) {
 #pragma unroll
     for (int g = 0; g < NA; ++g)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vmax[g][r] = a.v[uint64_t(argm[g][r]) * a.kv_ld + uint64_t(kvh) * a.hd + dim];
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t key = argm[g][r];
+        if constexpr (!OVER) {
+          vmax[g][r] = a.v[uint64_t(key) * a.kv_ld + uint64_t(kvh) * a.hd + dim];
+        } else {
+          const int8_t* c = src.v - l * 16 + uint64_t(key / 64) * 4 * kOp + (key / 16 % 4 * 16 + (l & 15)) * 16 + key % 16;
+          vmax[g][r] = c[0] + c[kOp] * 256 + c[2 * kOp] * 65536 + int32_t(kC3);
+          if (vw[key / 64]) vmax[g][r] += int32_t(uint32_t(c[3 * kOp]) << 24) + int32_t(kC4 - kC3);
+        }
+      }
     // sum of v' over the window's substeps: lane group g takes every fourth one,
     // eight loads at a time (one after the other they cost more than the products)
     for (uint32_t k = ks0 + (l >> 4); k < ks1; k += 32) {
@@ -795,14 +806,19 @@ __global__ __launch_bounds__(512) void k_attn_wsum_mfma(AttnMfmaArgs a) {
     }
   }
 }
-template <int GB>
-void launch_wsum(const AttnMfmaArgs& m, uint64_t nkv, hipStream_t s) {
+template <int GB, bool OVER>
+void launch_wsum_over(const AttnMfmaArgs& m, uint64_t nkv, hipStream_t s) {
   constexpr uint32_t lds = std::max(WsumShape<GB, 3>::lds, WsumShape<GB, 4>::lds);
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_wsum_mfma<GB>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_wsum_mfma<GB, OVER>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   (void)attr;
   const dim3 grid(unsigned(nkv), unsigned((m.crow_used + 15) / 16), unsigned((m.hd / 16 + 7) / 8));
-  hipLaunchKernelGGL((k_attn_wsum_mfma<GB>), grid, dim3(512), lds, s, m);
+  hipLaunchKernelGGL((k_attn_wsum_mfma<GB, OVER>), grid, dim3(512), lds, s, m);
+}
+template <int GB>
+void launch_wsum(const AttnMfmaArgs& m, uint64_t nkv, hipStream_t s) {
+  if (m.v_overwritten) launch_wsum_over<GB, true>(m, nkv, s);
+  else launch_wsum_over<GB, false>(m, nkv, s);
 }
 // Score rows (int32) of one chunk of queries. At 5000 queries, 8 heads of 256:
 // 128 MB 1.03 ms, 256 MB 0.97 ms (four chunks), 384 MB 0.93 ms, 64 MB 1.3 ms
@@ -873,6 +889,10 @@ bool attn_mfma_plan(const AttnArgs& a, AttnMfmaArgs& m) {
   m.crow = attn_chunk_rows(a);
   m.v = a.v;
   m.kv_ld = a.kv_ld;
+  // (V is read again while outputs are written, unless they share memory: its limbs then)
+  const uintptr_t v0 = reinterpret_cast<uintptr_t>(a.v), o0 = reinterpret_cast<uintptr_t>(a.out);
+  const uint64_t v_bytes = ((a.avail - 1) * a.kv_ld + nkv * a.hd) * 4, o_bytes = ((a.n_queries - 1) * a.out_ld + nh * a.hd) * 4;
+  m.v_overwritten = v0 < o0 + o_bytes && o0 < v0 + v_bytes;
   m.out = a.out;
   m.out_ld = a.out_ld;
   auto carve = [&](uint64_t bytes) {

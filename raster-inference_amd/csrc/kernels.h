@@ -319,6 +319,7 @@ struct AttnMfmaArgs {
   uint32_t* vwide;  // per KV head, 256 head dims and key substep: the V limbs take the four-limb split
   const int32_t* v;
   uint64_t kv_ld;
+  int v_overwritten;  // out shares memory with v
   // the chunk of queries [t0, t0 + crow_used) whose scores (crow rows per
   // head) are in the work area
   uint64_t t0, crow, crow_used;

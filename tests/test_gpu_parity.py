@@ -297,6 +297,19 @@ def test_attention_causal_chunks_of_queries(ctx, n, nh, nkv, hd, window, edges, 
     check_attention_rows(out.numpy(), q, k, v, {x for x in picks if x < n}, nh, nkv, hd, window)
 
 
+@pytest.mark.parametrize("n,nh,hd,over,wide", [(300, 2, 64, "v", False), (1100, 4, 128, "v", True), (700, 2, 320, "v", True),
+                                             (300, 2, 64, "q", False), (300, 2, 64, "k", False)])
+def test_attention_in_place(ctx, n, nh, hd, over, wide):
+    """The outputs may take the place of the queries, the keys or the values."""
+    q, k, v = attention_rows(n + hd, n, n, nh, nh, hd)
+    if wide:
+        v[4], v[130, 3], v[600, nh * hd - 1] = 1 << 24, -(1 << 31), (1 << 31) - 1
+    dev = {"q": ctx.to_device(q), "k": ctx.to_device(k), "v": ctx.to_device(v)}
+    ctx.attention(dev["q"], dev["k"], dev["v"], n, n, nh, nh, hd, 0, dev[over])
+    got = dev[over].numpy()
+    check_attention_rows(got, q, k, v, {0, 4, 9, 10, 15, 131, n // 2, n - 1}, nh, nh, hd, 0)
+
+
 @pytest.mark.parametrize("warm,warm_window,n", [(3712, 0, 3584), (700, 48, 700), (5000, 0, 4500)])
 def test_attention_recorded_after_a_longer_call(warm, warm_window, n):
     """A call of at least as many rows, windowed or not, leaves scratch that a recorded call of fewer rows fits:
