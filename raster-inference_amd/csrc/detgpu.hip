@@ -1073,6 +1073,7 @@ struct det_session {
   template <class T>
   T* alloc(uint64_t n) {
     if (!sizing) {
+      if (places.empty()) throw Status(3, "session buffer outside build()");
       uint8_t* p = places.back();
       places.pop_back();
       return reinterpret_cast<T*>(p);
