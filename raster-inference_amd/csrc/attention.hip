@@ -7,7 +7,7 @@
 //   x = c0 + 256 c1 + 65536 c2 + C3,               C3 = 32896    (x in [-2^23, 2^23)),
 //   x = c0 + 256 c1 + 65536 c2 + 2^24 c3 + C4,     C4 = 8421504,
 // c_j the signed bytes of (x + 2^23) ^ 0x808080 or of x ^ 0x808080. The groups
-// are one row of Q or K (its head dims), and 64 keys of V. A softmax weight w
+// are one row of Q or K (its head dims), and 64 keys x 256 dims of V. A softmax weight w
 // lies in [0, 65536]; only the first argmax row can hold 65536 (every other
 // weight is at most half), so w is split as two bytes of w ^ 0x8080 plus 32896
 // with that row clamped to 65535, and the clamped unit goes with the residual
@@ -821,9 +821,10 @@ void launch_wsum(const AttnMfmaArgs& m, uint64_t nkv, hipStream_t s) {
   else launch_wsum_over<GB, false>(m, nkv, s);
 }
 // Score rows (int32) of one chunk of queries. At 5000 queries, 8 heads of 256:
-// 128 MB 1.03 ms, 256 MB 0.97 ms (four chunks), 384 MB 0.93 ms, 64 MB 1.3 ms
-// (each chunk ends on a partly filled device); 256 MB keeps the whole work
-// area within its bound up to 16000 rows of that shape.
+// 64 MB 1.29 ms, 128 MB 0.94 ms, 256 MB 0.84 ms (four chunks), 384 MB 0.86 ms;
+// 3500 queries 0.64, 0.49, 0.46 and 0.41 ms (each chunk ends on a partly filled
+// device). 256 MB keeps the whole work area within its bound up to 16000 rows
+// of that shape.
 constexpr uint64_t kScoreBytes = uint64_t(256) << 20;
 
 // Keys of a score row: every key, or with a window the union window of 32
