@@ -263,7 +263,8 @@ __device__ __forceinline__ void score_block(const AttnMfmaArgs& a, int8_t* ring,
       if (c >= uint32_t(SLOTS)) c = SLOTS - 1;  // (spare slots copy the last block again)
       uint64_t J = j0 + uint64_t(st) * KS + c / (NSUB * NL);
       if (J >= j1) J = j1 - 1;
-      ring_copy(kb + ((J * NSUB + c / NL % NSUB) * 4 + c % NL) * kOp + l * 16, ring + ((st % kScoreStages) * SLOTS + c) * kOp);
+      ring_copy(kb + ((J * NSUB + c / NL % NSUB) * 4 + c % NL) * kOp + l * 16,
+                ring + ((st % kScoreStages) * SLOTS + c) * kOp);
     }
   };
   copy_stage(0);
@@ -353,7 +354,7 @@ void launch_scores_nw(const AttnMfmaArgs& m, uint64_t nkv, hipStream_t s) {
   // and registers leave room for two) and one block on every other CU beyond
   // (128 KB of ring, 32 KB of query operands per wave to load first). Never
   // less than eight tiles left 100 queries of 4 heads of 512 on four blocks:
-  // 17.0 us, now 5; 8/2 heads of 256 at 300 queries 15.8 -> 7.2.
+  // 17.0 us, now 6.8; 8/2 heads of 256 at 300 queries 15.8 -> 7.4.
   constexpr uint64_t want = NSUB <= 4 ? 512 : 128;
   while (span > 1 && all < want * span) span /= 2;
   const dim3 grid(unsigned(nkv), unsigned(y), unsigned(std::max<uint64_t>((most + span - 1) / span, 1)));
@@ -372,7 +373,7 @@ void launch_scores_nsub(const AttnMfmaArgs& m, uint64_t nkv, hipStream_t s) {
 // that share a score row's first key. A row's scores, then its exp terms, are
 // kept in LDS, so that the three passes are rolled loops (unrolled over
 // registers they were 66 to 130 KB of code, more than the instruction cache of
-// two CUs, and cost 25-35 % on windows of 512). Terms 16 or more below the
+// two CUs: 46 us against now 38 for 1000 rows of 16 heads in windows of 512). Terms 16 or more below the
 // maximum are zero exactly, and 64 keys that have only such terms skip the exp
 // series and the weights (rows of 256 normalised dims have scores of standard
 // deviation 16).
@@ -586,12 +587,13 @@ void launch_softmax(const AttnMfmaArgs& m, uint64_t nh, hipStream_t s) {
 // 72 queries x 79 substeps). A window that holds a four-limb V substep takes a
 // ring of three stages with all four limbs (read from global memory when they
 // came, they cost a third of the time). The rows' extras and the argmax rows'
-// values are read ahead of the loop: behind it, with a layer's caches cold, the
-// chain of two loads was 4 us of 15 at 120 queries. 32 queries per block halve
-// the V traffic but leave half the blocks: 1643 queries 172 us for the whole
-// attention against 158, 5000 queries the same. Lane l holds, in component r,
-// query 4 (l >> 4) + r and dim 16 D + (l & 15). Blocks of the longest windows
-// come first. grid (kv heads, query tiles, ceil(dim tiles / 8)), block 512.
+// values are read ahead of the loop, and the first stage's copies come before
+// any other load: with the chain of two loads behind the loop the kernel took
+// 15.0 us in a layer of 120 rows, whose caches are cold, now 10.0. 32 queries
+// per block halve the V traffic but leave half the blocks: 1643 queries 172 us
+// for the whole attention against 158, 5000 queries the same. Lane l holds, in
+// component r, query 4 (l >> 4) + r and dim 16 D + (l & 15). Blocks of the
+// longest windows come first. grid (kv heads, query tiles, ceil(dim tiles / 8)), block 512.
 template <int GB, int VL>
 struct WsumShape {
   static constexpr int NA = GB;                 // weight tiles, one per head
@@ -600,7 +602,8 @@ struct WsumShape {
   static constexpr int NB = VL == 3 ? 4 : 3;      // stages
   static constexpr uint32_t lds = NB * STAGE * kOp;
 };
-// A block's sources: the wave's weight halves and V limbs (this lane's bytes) of substep 0 of the score rows and of the cache.
+// A wave's sources, this lane's bytes: its weight halves at the start of the
+// score rows, its V limbs of the cache's first substep.
 template <int RPW>
 struct WsumSrc {
   const int8_t* w[RPW];
@@ -892,7 +895,8 @@ bool attn_mfma_plan(const AttnArgs& a, AttnMfmaArgs& m) {
   m.kv_ld = a.kv_ld;
   // (V is read again while outputs are written, unless they share memory: its limbs then)
   const uintptr_t v0 = reinterpret_cast<uintptr_t>(a.v), o0 = reinterpret_cast<uintptr_t>(a.out);
-  const uint64_t v_bytes = ((a.avail - 1) * a.kv_ld + nkv * a.hd) * 4, o_bytes = ((a.n_queries - 1) * a.out_ld + nh * a.hd) * 4;
+  const uint64_t v_bytes = ((a.avail - 1) * a.kv_ld + nkv * a.hd) * 4;
+  const uint64_t o_bytes = ((a.n_queries - 1) * a.out_ld + nh * a.hd) * 4;
   m.v_overwritten = v0 < o0 + o_bytes && o0 < v0 + v_bytes;
   m.out = a.out;
   m.out_ld = a.out_ld;

@@ -215,10 +215,10 @@ namespace {
 void abort_capture(det_ctx* ctx) {
   if (!ctx || !ctx->capturing) return;
   ctx->capturing = false;
-  ctx->recorded.clear();
   hipGraph_t g = nullptr;
   (void)hipStreamEndCapture(ctx->stream, &g);
   if (g) (void)hipGraphDestroy(g);
+  ctx->recorded.clear();
 }
 
 template <class F>
