@@ -1060,13 +1060,16 @@ struct det_session {
   // A session is about forty buffers, and an allocation and a free of each
   // cost more than the first decode steps: build() runs the code that
   // allocates them twice, first to take their sizes and then to hand out their
-  // places in a few device allocations of exactly the size of what they hold.
-  // Buffers of up to 1 MB share allocations of up to 1 MB, which the runtime
-  // serves from blocks it keeps (1.5 us with the release; from 2 MB on 14 us,
-  // and 250 us when one of the two goes to the driver); the larger ones share
-  // one. First layer prefill of a new scratch, 60 / 250 / 1200 rows: 500 / 720
-  // / 1570 us, with one allocation per larger buffer 640 / 990 / 1940; at 16
-  // rows and in a head's 380 and 160 us against 450 and 310 in one allocation.
+  // places in a few device allocations of the size of what they hold.
+  // Buffers of up to 1 MB share allocations of 1.25 MB, which the runtime
+  // serves from blocks that it keeps (1.5 us with the release; from 2 MB on 14
+  // us, and 250 us when one of the two goes to the driver) and that hold
+  // nothing else (in pieces of blocks shared with other memory the two-layer
+  // request of 16 + 16 tokens took 0.5 % longer, 1887 against 1877 us); the
+  // larger ones share one. First layer prefill of a new scratch, 60 / 250 /
+  // 1200 rows: 500 / 720 / 1570 us, with one allocation per larger buffer 640
+  // / 990 / 1940; at 16 rows and in a head's 380 and 160 us against 450 and
+  // 310 with one allocation of everything.
   bool sizing = false;
   std::vector<uint64_t> sizes;
   std::vector<uint8_t*> places;
@@ -1086,6 +1089,7 @@ struct det_session {
   }
   template <class F>
   void build(F&& cuts) {
+    constexpr uint64_t kSmall = uint64_t(1) << 20, kBlock = uint64_t(5) << 18;
     sizing = true;
     cuts();
     sizing = false;
@@ -1095,7 +1099,7 @@ struct det_session {
     auto flush = [&] {
       if (held.empty()) return;
       void* p = nullptr;
-      HIPC(hipMalloc(&p, bytes));
+      HIPC(hipMalloc(&p, std::max(bytes, kBlock)));
       owned.push_back(p);
       uint8_t* at = static_cast<uint8_t*>(p);
       for (const size_t i : held) {
@@ -1105,11 +1109,10 @@ struct det_session {
       held.clear();
       bytes = 0;
     };
-    constexpr uint64_t kSmall = uint64_t(1) << 20;
     for (const bool small : {true, false}) {
       for (size_t i = 0; i < sizes.size(); ++i) {
         if ((sizes[i] <= kSmall) != small) continue;
-        if (small && bytes + sizes[i] > kSmall) flush();
+        if (small && bytes + sizes[i] > kBlock) flush();
         if (__builtin_add_overflow(bytes, sizes[i], &bytes)) throw Status(3, "session buffers: out of memory");
         held.push_back(i);
       }
